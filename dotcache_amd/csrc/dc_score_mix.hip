@@ -7,6 +7,7 @@
 // s * (codes . q_g) + b * sum(q_g) for affine pages, s * ((codes - zp) . q_g)
 // for symmetric pages, fp32 escape rows for M3 pages.
 #include "dc_common.h"
+#include "dc_unpack.h"
 
 namespace dc {
 
@@ -85,8 +86,162 @@ __global__ void __launch_bounds__(256) score_pages_kernel(dc_pool pool, const in
   }
 }
 
-// grid.x = query row (group * n_queries + q), grid.y = channel block; one
-// thread per channel, looping over the pages of the row's group
+// ---- mix over 16-channel slices -------------------------------------------
+//
+// out[q, c] (+)= sum over tokens of w[q, t] V[t, c] for 16 channels c0 ..
+// c0 + 15 and QB queries per block of kMixWaves wavefronts.  The tokens of
+// the group's pages are cut into units of 64; wave w takes units w, w +
+// kMixWaves, ..., one token per lane, so code words and weights are read
+// contiguously and every lane keeps QB x 16 sums in registers.  The lanes'
+// sums meet in a butterfly that halves them at each step, the waves' in LDS,
+// in a fixed order.  What bounds it at these sizes is latency: the chain page
+// id -> descriptor -> words is walked once per 64 units (lane j holds unit
+// j's page), and unit j + 1's words are in flight while unit j is summed.
+// One block per slice rather than per query head: a single query's 128
+// channels run on 8 CUs instead of one, 1024 tokens at a time.  4096 tokens of
+// 4-bit pages at head_dim 128: one query 1139 -> 10.9 us, 8 groups of 3
+// queries 1149 -> 11.5 us (8 waves: 14.2; 8 waves with blocks of 4 queries:
+// 16.6 us; a third unit in flight does not fit 1024 threads' registers).
+template <int QB, int kMixWaves>
+__global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
+    dc_pool pool, const int32_t* __restrict__ page_ids, const int32_t* __restrict__ token_offsets, int32_t n_pages,
+    const int32_t* __restrict__ group_pages, int32_t n_queries, const float* __restrict__ weights,
+    int64_t weights_stride, float* out, int32_t accumulate) {
+  __shared__ float part[kMixWaves][QB * 16];
+  const dc_page_geometry geo = pool.geometry;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int32_t grp = blockIdx.z, q0 = blockIdx.y * QB, c0 = blockIdx.x * 16, C = geo.page_capacity;
+  const int nq = n_queries - q0 < QB ? n_queries - q0 : QB;
+  int32_t i0 = 0, i1 = n_pages;
+  if (group_pages) {
+    i0 = group_pages[grp] < 0 ? 0 : group_pages[grp];
+    i1 = group_pages[grp + 1] > n_pages ? n_pages : group_pages[grp + 1];
+  }
+  const float* w0 = weights + (int64_t(grp) * n_queries + q0) * weights_stride;
+  const int32_t upp = (C + 63) >> 6;  // units per page
+  const int64_t units = i1 > i0 ? int64_t(i1 - i0) * upp : 0;
+
+  float acc[QB][16];
+#pragma unroll
+  for (int q = 0; q < QB; ++q)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[q][i] = 0.f;
+
+  struct Unit {  // one unit's loads: raw words, scale, bias, weights of this lane's token
+    uint32_t r[16];
+    float s, b, w[QB];
+    int kind, shift;
+    bool live;
+  };
+  for (int64_t base = wave; base < units; base += 64 * kMixWaves) {
+    // lane j: the page of unit base + kMixWaves j
+    const int64_t u = base + int64_t(kMixWaves) * lane;
+    int32_t block = 0, info = 0, off = 0, sub = 0;
+    if (u < units) {
+      const int32_t i = i0 + int32_t(u / upp);
+      sub = int32_t(u - int64_t(i - i0) * upp) * 64;
+      const int32_t pid = page_ids[i];
+      off = token_offsets[i] + sub;
+      if (pid >= 0 && pid < pool.n_descs) {
+        const dc_page_desc d = pool.descs[pid];
+        const BlobLayout L = blob_layout(d.format, d.bits, geo);
+        const int32_t T = (d.tokens < C ? d.tokens : C) - sub;
+        if ((int64_t(d.block) << 8) + L.total <= pool.arena_bytes && T > 0) {
+          block = int32_t(d.block);
+          info = (T < 64 ? T : 64) | int32_t(d.format) << 8 | int32_t(d.bits) << 16;
+        }
+      }
+    }
+    const int64_t left = (units - base + kMixWaves - 1) / kMixWaves;
+    const int n = left < 64 ? int(left) : 64;
+
+    auto load = [&](int j, Unit& x) __attribute__((always_inline)) {
+      const int32_t inf = __builtin_amdgcn_readlane(info, j);
+      dc_page_desc d{};
+      d.block = uint32_t(__builtin_amdgcn_readlane(block, j));
+      d.format = uint8_t(inf >> 8);
+      d.bits = uint8_t(inf >> 16);
+      const int32_t T = inf & 0xff, o = __builtin_amdgcn_readlane(off, j), t0 = __builtin_amdgcn_readlane(sub, j);
+      x.kind = T > 0 ? chunk_kind(d.format, d.bits) : CK_NONE;
+      x.s = 1.f;
+      x.b = 0.f;
+      if (x.kind == CK_NONE) return;
+      const BlobLayout L = blob_layout(d.format, d.bits, geo);
+      const Chunk16 ck = chunk16_at(d.format, d.bits, geo, L, c0);
+      x.shift = ck.shift;
+      // (a lane past the page's tokens reads its last token, and adds nothing)
+      x.live = lane < T;
+      const uint32_t t = uint32_t(t0 + (lane < T ? lane : T - 1));
+      const uint8_t* blob = blob_ptr(pool.arena, d);
+      load_chunk16(x.kind, blob + ck.word + t * ck.word_step, x.r);
+      if (is_m0(d.format) || d.format == DC_FMT_M3_I8) {
+        x.s = __half2float(*reinterpret_cast<const __half*>(blob + ck.scale + t * ck.scale_step));
+        if (d.format == DC_FMT_M0_AFFINE) x.b = __half2float(*reinterpret_cast<const __half*>(blob + ck.bias + t * ck.scale_step));
+        if (d.format == DC_FMT_M0_SYMMETRIC) x.b = -float((1 << (d.bits - 1)) - 1) * x.s;
+      }
+#pragma unroll
+      for (int q = 0; q < QB; ++q)
+        x.w[q] = q < nq && x.live ? w0[int64_t(q) * weights_stride + o + lane] : 0.f;
+    };
+    auto sum = [&](const Unit& x) __attribute__((always_inline)) {
+      for_chunk_kind(x.kind, [&](auto k) __attribute__((always_inline)) {
+        float v[16];
+        values16<decltype(k)::value>(x.r, x.shift, x.s, x.b, v);
+        if (!x.live) return;
+#pragma unroll
+        for (int q = 0; q < QB; ++q)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[q][i] = fmaf(x.w[q], v[i], acc[q][i]);
+      });
+    };
+    Unit A, B;
+    load(0, A);
+    for (int j = 0; j < n; j += 2) {
+      if (j + 1 < n) load(j + 1, B);
+      sum(A);
+      if (j + 1 >= n) break;
+      if (j + 2 < n) load(j + 2, A);
+      sum(B);
+    }
+  }
+
+  // Lanes: at each step a lane keeps one half of its sums and adds its
+  // partner's copy of that half, so N sums take N - 1 exchanges; once one
+  // sum is left the remaining steps add whole copies.  With N = 16 QB sums
+  // the lane's sum is number (lane >> (6 - log2 N)) counted from the top bit.
+  float* f = &acc[0][0];
+  int idx = 0;
+#pragma unroll
+  for (int step = 0; step < 6; ++step) {
+    const int o = 32 >> step, n = (16 * QB) >> step;  // sums before this step
+    if (n > 1) {
+      const bool up = (lane & o) != 0;
+      idx = 2 * idx + (up ? 1 : 0);
+#pragma unroll
+      for (int i = 0; i < n / 2; ++i) {
+        const float send = up ? f[i] : f[i + n / 2];
+        const float keep = up ? f[i + n / 2] : f[i];
+        f[i] = keep + __shfl_xor(send, o, 64);
+      }
+    } else {
+      f[0] += __shfl_xor(f[0], o, 64);
+    }
+  }
+  part[wave][idx] = f[0];  // (lanes that share a sum write the same value)
+  __syncthreads();
+  const int k = threadIdx.x;
+  if (k < 16 * QB && k / 16 < nq) {
+    float total = part[0][k];
+#pragma unroll
+    for (int w = 1; w < kMixWaves; ++w) total += part[w][k];
+    float* o = out + (int64_t(grp) * n_queries + q0 + k / 16) * geo.head_dim + c0 + k % 16;
+    *o = accumulate ? *o + total : total;
+  }
+}
+
+// Geometries whose groups or rows are no multiple of 16 channels: grid.x =
+// query row (group * n_queries + q), grid.y = channel block; one thread per
+// channel, looping over the pages of the row's group
 // [group_pages[g], group_pages[g + 1]) (every page without group_pages) and
 // their tokens.
 __global__ void __launch_bounds__(256) mix_pages_kernel(dc_pool pool, const int32_t* __restrict__ page_ids,
@@ -145,6 +300,21 @@ static int mix_launch(const dc_pool& pool, const int32_t* page_ids, const int32_
   if (n_queries == 0) return DC_OK;
   if (!weights || !out || (n_pages > 0 && (!page_ids || !token_offsets || !pool.arena || !pool.descs)))
     return dc::fail(DC_EINVAL, "%s: null pointer", who);
+  if (dc::chunk16_geometry(pool.geometry) && n_groups <= 65535 && n_queries <= 65535) {
+    // (blocks of as many queries as there are, up to 4: 64 sums per lane)
+    // blocks of 2 queries (32 sums per lane) where there are two
+    const int qb = n_queries >= 2 ? 2 : 1;
+    const dim3 grid(uint32_t(pool.geometry.head_dim / 16), uint32_t((n_queries + qb - 1) / qb), uint32_t(n_groups));
+#define DC_MIX(QB_, W_)                                                                                              \
+  hipLaunchKernelGGL((dc::mix_slices_kernel<QB_, W_>), grid, dim3(64 * W_), 0, stream, pool, page_ids,               \
+                     token_offsets, n_pages, group_pages, n_queries, weights, weights_stride, out, accumulate)
+    if (qb == 1)
+      DC_MIX(1, 16);
+    else
+      DC_MIX(2, 16);
+#undef DC_MIX
+    return dc::check_hip(hipGetLastError(), who);
+  }
   const uint32_t cblocks = uint32_t((pool.geometry.head_dim + 255) / 256);
   hipLaunchKernelGGL(dc::mix_pages_kernel, dim3(uint32_t(n_groups) * uint32_t(n_queries), cblocks), dim3(256), 0,
                      stream, pool, page_ids, token_offsets, n_pages, group_pages, n_queries, weights, weights_stride,

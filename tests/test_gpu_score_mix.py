@@ -1,0 +1,64 @@
+"""``dc_score_pages`` / ``dc_mix_pages`` over every page format and the sizes
+where their tiles end: token counts around 64, page capacities below and
+above it, head_dims that are one or several 16-channel slices or no multiple
+of 16, and query counts around a block's 4."""
+import numpy as np
+import pytest
+
+from oracle import dotcache_oracle as O
+from tests.helpers import hard_values, to_product_page
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [dict(bits=2), dict(bits=3), dict(bits=3, scheme="symmetric"), dict(bits=4), dict(bits=4, scheme="symmetric"),
+           dict(bits=8), dict(bits=8, scheme="symmetric"), dict(mode="M3"), dict(mode="M3", escape_dtype="float32"),
+           dict(mode="M3", escape_dtype="int8")]
+
+
+def _groups(rng, hd, gs, fmt, lens, tpp, kind, layout):
+    pages = [O.encode_pages(hard_values(rng, n, hd), tokens_per_page=tpp, head_dim=hd, group_size=gs, kind=kind,
+                            layout=layout, **fmt) for n in lens]
+    return pages, [[to_product_page(p) for p in g] for g in pages]
+
+
+@pytest.mark.parametrize("fmt", FORMATS, ids=lambda f: "-".join(str(v) for v in f.values()))
+@pytest.mark.parametrize("hd,gs,tpp,Q,lens,layout", [
+    (128, 32, 64, 1, [1], "group_major"),
+    (128, 32, 64, 3, [63, 63], "group_major"),
+    (64, 16, 32, 4, [97, 97, 97], "group_major"),
+    (96, 32, 100, 5, [257, 257], "token_major"),
+    (256, 64, 128, 9, [700], "group_major"),
+    (80, 48, 64, 2, [130], "group_major"),
+    (48, 24, 64, 2, [70], "group_major"),
+])
+def test_grouped_logits_weights_and_output(fmt, hd, gs, tpp, Q, lens, layout):
+    from dotcache_amd.backends import decode_grouped_multiquery_step_prepared_hip_tensor as grouped
+
+    print(f"grouped {fmt} hd {hd} gs {gs} page {tpp} Q {Q} {lens} {layout}", flush=True)
+    rng = np.random.default_rng(hd + tpp + Q)
+    q = (rng.normal(size=(len(lens), Q, hd)) / np.sqrt(hd)).astype(np.float32)
+    okp, kp = _groups(rng, hd, gs, fmt, lens, tpp, "K", layout)
+    ovp, vp = _groups(rng, hd, gs, fmt, lens, tpp, "V", layout)
+    logits, weights, out = (t.cpu().numpy() for t in grouped(list(q), kp, vp))
+    for g in range(len(lens)):
+        want = O.decode_multi_query_step(q[g], okp[g], ovp[g])
+        # fp32 sums of up to 256 products of |q| < 0.5 and |k| < 60 (logits),
+        # of 700 weights that sum to 1 and |v| < 60 (output): both orders stay
+        # within n 2^-24 of the summed magnitudes, under 1e-4
+        np.testing.assert_allclose(logits[g], want[0], atol=1e-4, rtol=1e-5)
+        np.testing.assert_allclose(weights[g], want[1], atol=1e-5, rtol=1e-4)
+        np.testing.assert_allclose(out[g], want[2], atol=1e-4, rtol=1e-4)
+
+
+def test_mix_keeps_infinities_of_valid_rows_only():
+    """An infinite value row makes its channels infinite, not NaN, also as a
+    page's last token."""
+    from dotcache_amd import attention_runtime as rt
+
+    rng = np.random.default_rng(3)
+    v = rng.normal(size=(37, 64)).astype(np.float32)
+    v[36, 5] = np.inf
+    page = to_product_page(O.encode_page(v, head_dim=64, group_size=32, kind="V", mode="M3", escape_dtype="float32"))
+    w = np.full(37, 1 / 37, dtype=np.float32)
+    got = rt.mix_page(w, page, backend="hip_mi355x")
+    assert np.isposinf(got[5]) and np.isfinite(np.delete(got, 5)).all()
