@@ -27,11 +27,12 @@ COMMON = [
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
 ]
-# dc_decode_mfma.hip: MFMA results in VGPRs (the VGPR form of the
+# dc_decode_mfma.hip, dc_score_mix.hip: MFMA results in VGPRs (the VGPR form of the
 # instruction) instead of AGPRs, so the score's per-group results and the
 # softmax rescale of the accumulators need no AGPR <-> VGPR copies.
 PER_FILE = {"dc_encode.hip": ["-ffp-contract=off"],
-            "dc_decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
+            "dc_decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+            "dc_score_mix.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 
 def _hipcc() -> str:

@@ -289,10 +289,14 @@ def _mix_tensor(weights, pool: DevicePagePool, ids: np.ndarray, out=None):
     return out
 
 
-def _softmax_(x) -> None:
-    st = _lib.lib().dc_softmax_rows(C.c_void_p(x.data_ptr()), x.shape[0], x.shape[1], x.stride(0),
-                                    C.c_void_p(current_stream_ptr()))
-    _lib.check(st, "dc_softmax_rows")
+def _softmax(x):
+    """Softmax of the rows of fp32 ``x [..., n]`` (contiguous) in a new tensor."""
+    y = _torch().empty_like(x)
+    n = x.shape[-1]
+    st = _lib.lib().dc_softmax_rows_to(C.c_void_p(x.data_ptr()), n, C.c_void_p(y.data_ptr()), n,
+                                       x.numel() // n if n else 0, n, C.c_void_p(current_stream_ptr()))
+    _lib.check(st, "dc_softmax_rows_to")
+    return y
 
 
 def score_page_hip(query_slice: np.ndarray | Any, page: PageLike, *, trace: ExecutionTrace | None = None) -> np.ndarray:
@@ -373,8 +377,7 @@ def decode_multi_query_step_hip_tensor(query_slices, key_pages, value_pages, *, 
         if c.numel() != n:
             raise ValueError("precomputed page logits must have shape [token_count]")
         logits[:, offsets[i]: offsets[i + 1]] = c.reshape(1, n)
-    weights = logits.clone()
-    _softmax_(weights)
+    weights = _softmax(logits)
     out = _mix_tensor(weights, vpool, vid)
     return logits, weights, out
 
@@ -454,8 +457,7 @@ def decode_grouped_multiquery_step_prepared_hip_tensor(query_groups, key_pages_b
     _lib.check(L.dc_score_pages_grouped(kpool.c_pool(), C.c_void_p(kids_d.data_ptr()), C.c_void_p(off_d.data_ptr()),
                                         C.c_void_p(grp_d.data_ptr()), G, len(kids), C.c_void_p(q.data_ptr()), Q,
                                         C.c_void_p(logits.data_ptr()), T, stream), "dc_score_pages_grouped")
-    weights = logits.clone()
-    _lib.check(L.dc_softmax_rows(C.c_void_p(weights.data_ptr()), G * Q, T, T, stream), "dc_softmax_rows")
+    weights = _softmax(logits)
     out = torch.empty((G, Q, hd), dtype=torch.float32, device=dev)
     _lib.check(L.dc_mix_pages_grouped(vpool.c_pool(), C.c_void_p(vids_d.data_ptr()), C.c_void_p(off_d.data_ptr()),
                                       C.c_void_p(gp_d.data_ptr()), G, len(vids), C.c_void_p(weights.data_ptr()), Q, T,

@@ -13,7 +13,8 @@ namespace dc {
 
 constexpr int kScoreQ = 8;  // queries scored per pass
 
-// grid.x = page index, grid.y = query chunk; one thread per token.  With
+// Geometries that 16-channel chunks do not tile: grid.x = page index, grid.y
+// = query chunk; one thread per token.  With
 // page_group, page i is scored against the queries of group page_group[i]
 // (queries [n_groups][n_queries][hd]) into logits rows
 // group * n_queries + q; without it every page belongs to group 0.
@@ -84,6 +85,101 @@ __global__ void __launch_bounds__(256) score_pages_kernel(dc_pool pool, const in
     for (int j = 0; j < kScoreQ; ++j)
       if (j < nq) logits[int64_t(q0 + j) * logits_stride + off + t] = acc[j];
   }
+}
+
+// ---- score over 64-token tiles --------------------------------------------
+//
+// One wavefront scores 64 tokens of a page, one per lane, for 4 NB queries:
+// the lane unpacks its token's 16-channel chunks (contiguous words across
+// the lanes) and v_mfma_f32_4x4x1 multiplies each channel with four queries
+// at once, the queries (one chunk of four per register) broadcast from the A
+// operand's blocks.  No value crosses lanes and the logits leave in token
+// order.  Products and sums are fp32.  A page's words are read once for 4 NB
+// queries; the next chunk's words fly while one is multiplied.  A launch of a
+// few thousand tokens is bound by its chain of dependent loads (id,
+// descriptor, words; four chunks in flight measured the same).  4096 tokens of
+// 4-bit pages at head_dim 128: one query 37.9 -> 7.4 us, 8 groups of 3
+// queries 54.8 -> 7.9 us.
+template <int NB>
+__global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int32_t* __restrict__ page_ids,
+                                                         const int32_t* __restrict__ token_offsets,
+                                                         const int32_t* __restrict__ page_group, int32_t n_groups,
+                                                         const float* __restrict__ queries_all, int32_t n_queries,
+                                                         float* __restrict__ logits_all, int64_t logits_stride,
+                                                         int32_t units_per_page) {
+  const dc_page_geometry geo = pool.geometry;
+  const int32_t i = blockIdx.x / units_per_page, t0 = int32_t(blockIdx.x - uint32_t(i) * units_per_page) * 64;
+  const int32_t q0 = blockIdx.y * 4 * NB, hd = geo.head_dim;
+  const int lane = threadIdx.x;
+  const int32_t grp = page_group ? page_group[i] : 0, pid = page_ids[i], off = token_offsets[i];
+  if (grp < 0 || grp >= n_groups || pid < 0 || pid >= pool.n_descs) return;
+  const dc_page_desc d = pool.descs[pid];
+  const BlobLayout L = blob_layout(d.format, d.bits, geo);
+  if ((int64_t(d.block) << 8) + L.total > pool.arena_bytes) return;
+  const int32_t T = (d.tokens < geo.page_capacity ? d.tokens : geo.page_capacity) - t0;
+  if (T <= 0) return;
+  const uint8_t* blob = blob_ptr(pool.arena, d);
+  const uint32_t t = uint32_t(t0 + (lane < T ? lane : T - 1));  // (lanes past the page repeat its last token)
+
+  // lane (b, r) of a query register: channel 16 k + b of query q0 + 4 n + r
+  const float* qp[NB];
+  bool q_live[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) {
+    const int32_t q = q0 + 4 * n + (lane & 3);
+    q_live[n] = q < n_queries;
+    qp[n] = queries_all + (int64_t(grp) * n_queries + (q_live[n] ? q : q0)) * hd + (lane >> 2);
+  }
+  f32x4v s0[NB], s1[NB];
+#pragma unroll
+  for (int n = 0; n < NB; ++n) s0[n] = s1[n] = f32x4v{0.f, 0.f, 0.f, 0.f};
+
+  struct Chunk {
+    uint32_t r[16];
+    float s, b, q[NB];
+    int shift;
+  };
+  const float zp = float((1 << (d.bits - 1)) - 1);
+  for_chunk_kind(chunk_kind(d.format, d.bits), [&](auto kind) __attribute__((always_inline)) {
+    constexpr int K = decltype(kind)::value;
+    auto load = [&](int32_t c0, Chunk& x) __attribute__((always_inline)) {
+      const Chunk16 ck = chunk16_at(d.format, d.bits, geo, L, c0);
+      load_chunk16(K, blob + ck.word + t * ck.word_step, x.r);
+      x.shift = ck.shift;
+      x.s = 1.f;
+      x.b = 0.f;
+      if constexpr (K != CK_F16 && K != CK_F32) {
+        x.s = __half2float(*reinterpret_cast<const __half*>(blob + ck.scale + t * ck.scale_step));
+        if (d.format == DC_FMT_M0_AFFINE)
+          x.b = __half2float(*reinterpret_cast<const __half*>(blob + ck.bias + t * ck.scale_step));
+        if (d.format == DC_FMT_M0_SYMMETRIC) x.b = -zp * x.s;
+      }
+#pragma unroll
+      for (int n = 0; n < NB; ++n) x.q[n] = qp[n][c0];
+    };
+    auto dot = [&](const Chunk& x) __attribute__((always_inline)) {
+      float v[16];
+      values16<K>(x.r, x.shift, x.s, x.b, v);
+#pragma unroll
+      for (int n = 0; n < NB; ++n) dot16(q_live[n] ? x.q[n] : 0.f, v, s0[n], s1[n]);
+    };
+    Chunk A, B;
+    load(0, A);
+    for (int32_t c0 = 0; c0 < hd; c0 += 32) {
+      if (c0 + 16 < hd) load(c0 + 16, B);
+      dot(A);
+      if (c0 + 16 >= hd) break;
+      if (c0 + 32 < hd) load(c0 + 32, A);
+      dot(B);
+    }
+  });
+  if (lane >= T) return;
+  float* logits = logits_all + (int64_t(grp) * n_queries + q0) * logits_stride + off + t0 + lane;
+#pragma unroll
+  for (int n = 0; n < NB; ++n)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (q0 + 4 * n + r < n_queries) logits[int64_t(4 * n + r) * logits_stride] = s0[n][r] + s1[n][r];
 }
 
 // ---- mix over 16-channel slices -------------------------------------------
@@ -286,6 +382,23 @@ static int score_launch(const dc_pool& pool, const int32_t* page_ids, const int3
   if (n_pages == 0 || n_queries == 0) return DC_OK;
   if (!page_ids || !token_offsets || !queries || !logits || !pool.arena || !pool.descs)
     return dc::fail(DC_EINVAL, "%s: null pointer", who);
+  const int32_t upp = (pool.geometry.page_capacity + 63) / 64;
+  if (dc::chunk16_geometry(pool.geometry) && int64_t(n_pages) * upp < (int64_t(1) << 31) && n_queries <= 65535) {
+    // (queries per pass over the words: as many as there are, up to 16)
+    const int nb = n_queries <= 4 ? 1 : n_queries <= 8 ? 2 : 4;
+    const dim3 grid(uint32_t(n_pages * upp), uint32_t((n_queries + 4 * nb - 1) / (4 * nb)));
+#define DC_SCORE(NB_)                                                                                              \
+  hipLaunchKernelGGL((dc::score_tiles_kernel<NB_>), grid, dim3(64), 0, stream, pool, page_ids, token_offsets, page_group, \
+                     n_groups, queries, n_queries, logits, logits_stride, upp)
+    if (nb == 1)
+      DC_SCORE(1);
+    else if (nb == 2)
+      DC_SCORE(2);
+    else
+      DC_SCORE(4);
+#undef DC_SCORE
+    return dc::check_hip(hipGetLastError(), who);
+  }
   const uint32_t qchunks = uint32_t((n_queries + dc::kScoreQ - 1) / dc::kScoreQ);
   hipLaunchKernelGGL(dc::score_pages_kernel, dim3(uint32_t(n_pages), qchunks), dim3(128), 0, stream, pool, page_ids,
                      token_offsets, page_group, n_groups, queries, n_queries, logits, logits_stride);
@@ -356,40 +469,78 @@ extern "C" int dc_mix_pages_grouped(dc_pool pool, const int32_t* page_ids, const
 
 namespace dc {
 
-// In-place softmax of each row (reference attention_reference.py:27-31):
-// exp(x - max) / sum, fp32, one block per row.
-__global__ void __launch_bounds__(256) softmax_rows_kernel(float* __restrict__ x, int32_t n_cols, int64_t stride) {
-  float* row = x + int64_t(blockIdx.x) * stride;
-  __shared__ float red[4];
+// Softmax of each row (reference attention_reference.py:27-31): exp(x - max)
+// / sum, fp32, one block of 1024 threads per row, from src to dst (which may
+// be the same row).  Up to kSoftmaxRegs columns per thread stay in registers
+// between the passes; longer rows are read again (from dst once the
+// exponentials are there).  Bound by latency at a few thousand columns: one
+// load round, two block reductions (24 rows of 4096: 11.8 -> 4.8 us; 256
+// threads walked the row three times).
+constexpr int kSoftmaxRegs = 8;
+__global__ void __launch_bounds__(1024) softmax_rows_kernel(const float* src, int64_t src_stride, float* dst,
+                                                            int64_t dst_stride, int32_t n_cols) {
+  const float* x = src + int64_t(blockIdx.x) * src_stride;
+  float* y = dst + int64_t(blockIdx.x) * dst_stride;
+  __shared__ float red[2][16];
+  const int tid = threadIdx.x;
+  float v[kSoftmaxRegs];
+#pragma unroll
+  for (int k = 0; k < kSoftmaxRegs; ++k) {  // (every load in flight: a clamped column, masked)
+    const int32_t i = tid + 1024 * k;
+    v[k] = x[i < n_cols ? i : n_cols - 1];
+  }
   float mx = -INFINITY;
-  for (int32_t i = threadIdx.x; i < n_cols; i += blockDim.x) mx = fmaxf(mx, row[i]);
+#pragma unroll
+  for (int k = 0; k < kSoftmaxRegs; ++k) mx = tid + 1024 * k < n_cols ? fmaxf(mx, v[k]) : mx;
+  for (int32_t i = tid + 1024 * kSoftmaxRegs; i < n_cols; i += 1024) mx = fmaxf(mx, x[i]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = mx;
+  if (tid % 64 == 0) red[0][tid / 64] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 16; ++w) mx = fmaxf(mx, red[0][w]);
   float sum = 0.f;
-  for (int32_t i = threadIdx.x; i < n_cols; i += blockDim.x) {
-    const float e = expf(row[i] - mx);
-    row[i] = e;
+#pragma unroll
+  for (int k = 0; k < kSoftmaxRegs; ++k) {
+    v[k] = expf(v[k] - mx);
+    sum += tid + 1024 * k < n_cols ? v[k] : 0.f;
+  }
+  for (int32_t i = tid + 1024 * kSoftmaxRegs; i < n_cols; i += 1024) {
+    const float e = expf(x[i] - mx);
+    y[i] = e;
     sum += e;
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-  if (threadIdx.x % 64 == 0) red[threadIdx.x / 64] = sum;
+  if (tid % 64 == 0) red[1][tid / 64] = sum;
   __syncthreads();
-  sum = red[0] + red[1] + red[2] + red[3];
-  for (int32_t i = threadIdx.x; i < n_cols; i += blockDim.x) row[i] = row[i] / sum;
+  sum = 0.f;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) sum += red[1][w];
+#pragma unroll
+  for (int k = 0; k < kSoftmaxRegs; ++k)
+    if (tid + 1024 * k < n_cols) y[tid + 1024 * k] = v[k] / sum;
+  for (int32_t i = tid + 1024 * kSoftmaxRegs; i < n_cols; i += 1024) y[i] = y[i] / sum;
 }
 
 }  // namespace dc
 
-extern "C" int dc_softmax_rows(float* x, int32_t n_rows, int32_t n_cols, int64_t stride, dc_stream_t stream) {
-  if (n_rows < 0 || n_cols < 0 || (n_rows > 0 && stride < n_cols)) return dc::fail(DC_EINVAL, "dc_softmax_rows: bad shape");
+static int softmax_launch(const float* src, int64_t src_stride, float* dst, int64_t dst_stride, int32_t n_rows,
+                          int32_t n_cols, dc_stream_t stream, const char* who) {
+  if (n_rows < 0 || n_cols < 0 || (n_rows > 0 && (src_stride < n_cols || dst_stride < n_cols)))
+    return dc::fail(DC_EINVAL, "%s: bad shape", who);
   if (n_rows == 0 || n_cols == 0) return DC_OK;
-  if (!x) return dc::fail(DC_EINVAL, "dc_softmax_rows: null pointer");
-  hipLaunchKernelGGL(dc::softmax_rows_kernel, dim3(uint32_t(n_rows)), dim3(256), 0, hipStream_t(stream), x, n_cols,
-                     stride);
-  return dc::check_hip(hipGetLastError(), "dc_softmax_rows launch");
+  if (!src || !dst) return dc::fail(DC_EINVAL, "%s: null pointer", who);
+  hipLaunchKernelGGL(dc::softmax_rows_kernel, dim3(uint32_t(n_rows)), dim3(1024), 0, hipStream_t(stream), src,
+                     src_stride, dst, dst_stride, n_cols);
+  return dc::check_hip(hipGetLastError(), who);
+}
+
+extern "C" int dc_softmax_rows(float* x, int32_t n_rows, int32_t n_cols, int64_t stride, dc_stream_t stream) {
+  return softmax_launch(x, stride, x, stride, n_rows, n_cols, stream, "dc_softmax_rows");
+}
+
+extern "C" int dc_softmax_rows_to(const float* x, int64_t x_stride, float* y, int64_t y_stride, int32_t n_rows,
+                                  int32_t n_cols, dc_stream_t stream) {
+  return softmax_launch(x, x_stride, y, y_stride, n_rows, n_cols, stream, "dc_softmax_rows_to");
 }

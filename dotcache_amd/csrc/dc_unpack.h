@@ -12,6 +12,7 @@
 #pragma once
 
 #include <type_traits>
+#include <utility>
 
 #include "dc_common.h"
 
@@ -130,6 +131,28 @@ __device__ __forceinline__ void values16(const uint32_t (&r)[16], int shift, flo
 #pragma unroll
     for (int j = 0; j < 16; ++j) v[j] = __builtin_bit_cast(float, r[j]);
   }
+}
+
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+// d[i] += a[i] * b per lane for the four rows i of block J of a (lanes 4 J ..
+// 4 J + 3, one row each), read by every lane: one fp32 multiply-add per
+// (row, lane), in 8 cycles (v_mfma_f32_4x4x1, A block J broadcast to all 16).
+template <int J>
+__device__ __forceinline__ f32x4v mfma4_bcast(float a, float b, f32x4v d) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, d, 4, J, 0);
+}
+
+// d += sum over i < 16 of block i of a times v[i]: 16 channels (or tokens) of
+// four rows against this lane's 16 values, in two chains (even i in d0, odd
+// in d1) so that no product waits for the one before it.
+template <int... I>
+__device__ __forceinline__ void dot16(float a, const float (&v)[16], f32x4v& d0, f32x4v& d1,
+                                      std::integer_sequence<int, I...>) {
+  ((I % 2 == 0 ? void(d0 = mfma4_bcast<I>(a, v[I], d0)) : void(d1 = mfma4_bcast<I>(a, v[I], d1))), ...);
+}
+__device__ __forceinline__ void dot16(float a, const float (&v)[16], f32x4v& d0, f32x4v& d1) {
+  dot16(a, v, d0, d1, std::make_integer_sequence<int, 16>{});
 }
 
 // fn(std::integral_constant<int, KIND>) for a wave-uniform kind.

@@ -242,6 +242,10 @@ int dc_mix_pages_grouped(dc_pool pool, const int32_t* page_ids, const int32_t* t
  * point that returns logits and weights. */
 int dc_softmax_rows(float* x /* device */, int32_t n_rows, int32_t n_cols, int64_t stride, dc_stream_t stream);
 
+/* The same softmax from x into y (the rows must be the same or disjoint). */
+int dc_softmax_rows_to(const float* x /* device */, int64_t x_stride, float* y /* device */, int64_t y_stride,
+                       int32_t n_rows, int32_t n_cols, dc_stream_t stream);
+
 /* Execution shortlist (reference dotcache/session_runtime.py:122-439).
  *
  * Per-page summaries of pages page_ids[0 .. n_pages) of a pool, from their

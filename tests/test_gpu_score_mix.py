@@ -62,3 +62,27 @@ def test_mix_keeps_infinities_of_valid_rows_only():
     w = np.full(37, 1 / 37, dtype=np.float32)
     got = rt.mix_page(w, page, backend="hip_mi355x")
     assert np.isposinf(got[5]) and np.isfinite(np.delete(got, 5)).all()
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 8192, 8193, 20000])
+def test_softmax_rows_in_place_and_out_of_place(n):
+    """Around a row's register columns (8 x 1024) and past them."""
+    import ctypes as C
+
+    import torch
+
+    from dotcache_amd import _lib
+
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n)
+    x = torch.randn((3, n + 5), generator=gen, device="cuda") * 4
+    want = torch.softmax(x[:, :n].double(), dim=-1)
+    y = torch.full((3, n), -1.0, device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    keep = x.clone()
+    assert _lib.lib().dc_softmax_rows_to(x.data_ptr(), n + 5, y.data_ptr(), n, 3, n, stream) == 0
+    assert torch.equal(x, keep)
+    # each weight: one exp (2 ulp), a sum of n terms in a tree of depth < 32, one division
+    assert float(((y - want).abs() / want).max()) < 40 * 2.0 ** -24 + 2e-7 * float((x - x.amax(-1, True)).abs().max())
+    assert _lib.lib().dc_softmax_rows(x.data_ptr(), 3, n, n + 5, stream) == 0
+    assert torch.equal(x[:, :n], y) and torch.equal(x[:, n:], keep[:, n:])
