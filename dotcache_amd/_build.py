@@ -15,7 +15,7 @@ from pathlib import Path
 PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 LIB = PKG / "libdotcache_hip.so"
-SOURCES = ["dc_abi.cpp", "dc_encode.hip", "dc_score_mix.hip", "dc_decode.hip", "dc_decode_mfma.hip", "dc_shortlist.hip",
+SOURCES = ["dc_abi.cpp", "dc_encode.hip", "dc_score_mix.hip", "dc_decode.hip", "dc_decode_tiles.hip", "dc_decode_mfma.hip", "dc_shortlist.hip",
            "dc_decode_noalloc.hip"]
 
 # -packed-fp32-ops: no v_pk_*_f32 anywhere in the device code.
@@ -27,11 +27,12 @@ COMMON = [
     "-fhip-fp32-correctly-rounded-divide-sqrt",
     "-Wall", "-Wno-unused-function", "-Wno-unused-result",
 ]
-# dc_decode_mfma.hip, dc_score_mix.hip: MFMA results in VGPRs (the VGPR form of the
+# dc_decode_mfma.hip, dc_decode_tiles.hip, dc_score_mix.hip: MFMA results in VGPRs (the VGPR form of the
 # instruction) instead of AGPRs, so the score's per-group results and the
 # softmax rescale of the accumulators need no AGPR <-> VGPR copies.
 PER_FILE = {"dc_encode.hip": ["-ffp-contract=off"],
             "dc_decode_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+            "dc_decode_tiles.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
             "dc_score_mix.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 

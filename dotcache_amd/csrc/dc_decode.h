@@ -56,6 +56,8 @@ __device__ __forceinline__ float wave_sum(float v) {
 int launch_decode(const DecodeArgs& a, hipStream_t stream);
 int decode_mfma_waves(const DecodeArgs& a);
 int launch_decode_generic(const DecodeArgs& a, hipStream_t stream);
+// Launches the tile kernel (dc_decode_tiles.hip) when the geometry fits it.
+int launch_decode_tiles(const DecodeArgs& a, hipStream_t stream, bool* launched);
 // Launches the MFMA kernel when every format in the pools' masks and the
 // geometry fit it; *launched tells the caller whether to fall back.
 int launch_decode_mfma(const DecodeArgs& a, hipStream_t stream, bool* launched);

@@ -1,11 +1,13 @@
 // Fused paged decode: score -> single-pass online softmax -> mix, straight
 // from compressed pages, plus the split-K log-sum-exp merge.
 //
-// This file holds the generic path, which reads every page format the pool
-// can hold (M0 affine / symmetric 2/3/4/8-bit, any group size, both layouts;
-// M3 fp16 / fp32 / int8) and up to kMaxQ GQA query heads per KV head.  The
-// MFMA fast path for the common formats lives in dc_decode_mfma.hip and is
-// chosen by dc_decode_paged when every page of the call fits it.
+// This file holds the kernel of last resort, which reads every page format
+// the pool can hold (M0 affine / symmetric 2/3/4/8-bit, any group size, both
+// layouts; M3 fp16 / fp32 / int8) and up to kMaxQ GQA query heads per KV head.
+// The MFMA path for the common formats lives in dc_decode_mfma.hip and is
+// chosen by dc_decode_paged when every page of the call fits it; other pages
+// take dc_decode_tiles.hip, and this kernel only where group_size or head_dim
+// is no multiple of 16.
 //
 // Semantics: reference dotcache/attention_runtime.py:260-315 (concatenate
 // page logits, one softmax over the whole context, mix every value page)
@@ -497,6 +499,8 @@ __global__ void __launch_bounds__(256) merge_kernel(const dc_merge_item* __restr
 }
 
 int launch_decode_generic(const DecodeArgs& a, hipStream_t stream) {
+  bool launched = false;
+  if (int rc = launch_decode_tiles(a, stream, &launched); rc || launched) return rc;
   hipLaunchKernelGGL(decode_generic_kernel, dim3(uint32_t(a.n_items)), dim3(kThreads), 0, stream, a);
   return check_hip(hipGetLastError(), "decode_generic_kernel launch");
 }

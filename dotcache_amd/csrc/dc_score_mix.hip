@@ -95,11 +95,11 @@ __global__ void __launch_bounds__(256) score_pages_kernel(dc_pool pool, const in
 // at once, the queries (one chunk of four per register) broadcast from the A
 // operand's blocks.  No value crosses lanes and the logits leave in token
 // order.  Products and sums are fp32.  A page's words are read once for 4 NB
-// queries; the next chunk's words fly while one is multiplied.  A launch of a
+// queries; the next chunks' words fly while one is multiplied.  A launch of a
 // few thousand tokens is bound by its chain of dependent loads (id,
-// descriptor, words; four chunks in flight measured the same).  4096 tokens of
-// 4-bit pages at head_dim 128: one query 37.9 -> 7.4 us, 8 groups of 3
-// queries 54.8 -> 7.9 us.
+// descriptor, words).  4096 tokens of 4-bit pages at head_dim 128: one query
+// 37.9 -> 5.6 us, 8 groups of 3 queries 54.8 -> 6.5 us (7.4 and 7.9 with scales
+// converted where they are loaded, which waits for each load).
 template <int NB>
 __global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int32_t* __restrict__ page_ids,
                                                          const int32_t* __restrict__ token_offsets,
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int
   const int32_t grp = page_group ? page_group[i] : 0, pid = page_ids[i], off = token_offsets[i];
   if (grp < 0 || grp >= n_groups || pid < 0 || pid >= pool.n_descs) return;
   const dc_page_desc d = pool.descs[pid];
-  const BlobLayout L = blob_layout(d.format, d.bits, geo);
+  const Blob32 L = blob32(d.format, d.bits, geo, num_groups(geo));
   if ((int64_t(d.block) << 8) + L.total > pool.arena_bytes) return;
   const int32_t T = (d.tokens < geo.page_capacity ? d.tokens : geo.page_capacity) - t0;
   if (T <= 0) return;
@@ -123,56 +123,17 @@ __global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int
 
   // lane (b, r) of a query register: channel 16 k + b of query q0 + 4 n + r
   const float* qp[NB];
-  bool q_live[NB];
 #pragma unroll
   for (int n = 0; n < NB; ++n) {
     const int32_t q = q0 + 4 * n + (lane & 3);
-    q_live[n] = q < n_queries;
-    qp[n] = queries_all + (int64_t(grp) * n_queries + (q_live[n] ? q : q0)) * hd + (lane >> 2);
+    // (a head past the last repeats the block's first: its sums are not stored)
+    qp[n] = queries_all + (int64_t(grp) * n_queries + (q < n_queries ? q : q0)) * hd + (lane >> 2);
   }
   f32x4v s0[NB], s1[NB];
 #pragma unroll
   for (int n = 0; n < NB; ++n) s0[n] = s1[n] = f32x4v{0.f, 0.f, 0.f, 0.f};
 
-  struct Chunk {
-    uint32_t r[16];
-    float s, b, q[NB];
-    int shift;
-  };
-  const float zp = float((1 << (d.bits - 1)) - 1);
-  for_chunk_kind(chunk_kind(d.format, d.bits), [&](auto kind) __attribute__((always_inline)) {
-    constexpr int K = decltype(kind)::value;
-    auto load = [&](int32_t c0, Chunk& x) __attribute__((always_inline)) {
-      const Chunk16 ck = chunk16_at(d.format, d.bits, geo, L, c0);
-      load_chunk16(K, blob + ck.word + t * ck.word_step, x.r);
-      x.shift = ck.shift;
-      x.s = 1.f;
-      x.b = 0.f;
-      if constexpr (K != CK_F16 && K != CK_F32) {
-        x.s = __half2float(*reinterpret_cast<const __half*>(blob + ck.scale + t * ck.scale_step));
-        if (d.format == DC_FMT_M0_AFFINE)
-          x.b = __half2float(*reinterpret_cast<const __half*>(blob + ck.bias + t * ck.scale_step));
-        if (d.format == DC_FMT_M0_SYMMETRIC) x.b = -zp * x.s;
-      }
-#pragma unroll
-      for (int n = 0; n < NB; ++n) x.q[n] = qp[n][c0];
-    };
-    auto dot = [&](const Chunk& x) __attribute__((always_inline)) {
-      float v[16];
-      values16<K>(x.r, x.shift, x.s, x.b, v);
-#pragma unroll
-      for (int n = 0; n < NB; ++n) dot16(q_live[n] ? x.q[n] : 0.f, v, s0[n], s1[n]);
-    };
-    Chunk A, B;
-    load(0, A);
-    for (int32_t c0 = 0; c0 < hd; c0 += 32) {
-      if (c0 + 16 < hd) load(c0 + 16, B);
-      dot(A);
-      if (c0 + 16 >= hd) break;
-      if (c0 + 32 < hd) load(c0 + 32, A);
-      dot(B);
-    }
-  });
+  score_row<NB>(d, geo, L, blob, t, [&](int32_t c0, int n) { return qp[n][c0]; }, s0, s1);
   if (lane >= T) return;
   float* logits = logits_all + (int64_t(grp) * n_queries + q0) * logits_stride + off + t0 + lane;
 #pragma unroll
@@ -195,9 +156,9 @@ __global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int
 // j's page), and unit j + 1's words are in flight while unit j is summed.
 // One block per slice rather than per query head: a single query's 128
 // channels run on 8 CUs instead of one, 1024 tokens at a time.  4096 tokens of
-// 4-bit pages at head_dim 128: one query 1139 -> 10.9 us, 8 groups of 3
-// queries 1149 -> 11.5 us (8 waves: 14.2; 8 waves with blocks of 4 queries:
-// 16.6 us; a third unit in flight does not fit 1024 threads' registers).
+// 4-bit pages at head_dim 128: one query 1139 -> 9.4 us, 8 groups of 3
+// queries 1149 -> 10.8 us (8 waves: 14.2 before, and 16.6 us with blocks of 4
+// queries; a third unit in flight does not fit 1024 threads' registers).
 template <int QB, int kMixWaves>
 __global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
     dc_pool pool, const int32_t* __restrict__ page_ids, const int32_t* __restrict__ token_offsets, int32_t n_pages,
@@ -207,6 +168,7 @@ __global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
   const dc_page_geometry geo = pool.geometry;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int32_t grp = blockIdx.z, q0 = blockIdx.y * QB, c0 = blockIdx.x * 16, C = geo.page_capacity;
+  const uint32_t groups = num_groups(geo);
   const int nq = n_queries - q0 < QB ? n_queries - q0 : QB;
   int32_t i0 = 0, i1 = n_pages;
   if (group_pages) {
@@ -225,8 +187,9 @@ __global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
 
   struct Unit {  // one unit's loads: raw words, scale, bias, weights of this lane's token
     uint32_t r[16];
-    float s, b, w[QB];
-    int kind, shift;
+    uint16_t s, b;
+    float w[QB];
+    int kind, format, bits, shift;
     bool live;
   };
   for (int64_t base = wave; base < units; base += 64 * kMixWaves) {
@@ -240,7 +203,7 @@ __global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
       off = token_offsets[i] + sub;
       if (pid >= 0 && pid < pool.n_descs) {
         const dc_page_desc d = pool.descs[pid];
-        const BlobLayout L = blob_layout(d.format, d.bits, geo);
+        const Blob32 L = blob32(d.format, d.bits, geo, groups);
         const int32_t T = (d.tokens < C ? d.tokens : C) - sub;
         if ((int64_t(d.block) << 8) + L.total <= pool.arena_bytes && T > 0) {
           block = int32_t(d.block);
@@ -259,30 +222,36 @@ __global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
       d.bits = uint8_t(inf >> 16);
       const int32_t T = inf & 0xff, o = __builtin_amdgcn_readlane(off, j), t0 = __builtin_amdgcn_readlane(sub, j);
       x.kind = T > 0 ? chunk_kind(d.format, d.bits) : CK_NONE;
-      x.s = 1.f;
-      x.b = 0.f;
+      x.format = d.format;
+      x.bits = d.bits;
       if (x.kind == CK_NONE) return;
-      const BlobLayout L = blob_layout(d.format, d.bits, geo);
+      const Blob32 L = blob32(d.format, d.bits, geo, groups);
       const Chunk16 ck = chunk16_at(d.format, d.bits, geo, L, c0);
-      x.shift = ck.shift;
+      x.shift = ck.shift();
       // (a lane past the page's tokens reads its last token, and adds nothing)
       x.live = lane < T;
-      const uint32_t t = uint32_t(t0 + (lane < T ? lane : T - 1));
+      const uint32_t tok = x.live ? lane : T - 1, t = uint32_t(t0) + tok;
       const uint8_t* blob = blob_ptr(pool.arena, d);
-      load_chunk16(x.kind, blob + ck.word + t * ck.word_step, x.r);
-      if (is_m0(d.format) || d.format == DC_FMT_M3_I8) {
-        x.s = __half2float(*reinterpret_cast<const __half*>(blob + ck.scale + t * ck.scale_step));
-        if (d.format == DC_FMT_M0_AFFINE) x.b = __half2float(*reinterpret_cast<const __half*>(blob + ck.bias + t * ck.scale_step));
-        if (d.format == DC_FMT_M0_SYMMETRIC) x.b = -float((1 << (d.bits - 1)) - 1) * x.s;
+      // Loads only: conversions wait until the unit is summed, or each load
+      // would be waited for where it was issued.
+      load_chunk16(x.kind, blob + ck.word() + t * ck.word_step, x.r);
+      if (x.kind != CK_F16 && x.kind != CK_F32) {
+        x.s = *reinterpret_cast<const uint16_t*>(blob + ck.scale + t * ck.scale_step);
+        // (no bias: the scale again, unused)
+        x.b = *reinterpret_cast<const uint16_t*>(blob + (d.format == DC_FMT_M0_AFFINE ? ck.bias : ck.scale) + t * ck.scale_step);
       }
 #pragma unroll
-      for (int q = 0; q < QB; ++q)
-        x.w[q] = q < nq && x.live ? w0[int64_t(q) * weights_stride + o + lane] : 0.f;
+      for (int q = 0; q < QB; ++q) x.w[q] = w0[int64_t(q < nq ? q : 0) * weights_stride + o + int32_t(tok)];
     };
     auto sum = [&](const Unit& x) __attribute__((always_inline)) {
       for_chunk_kind(x.kind, [&](auto k) __attribute__((always_inline)) {
-        float v[16];
-        values16<decltype(k)::value>(x.r, x.shift, x.s, x.b, v);
+        constexpr int K = decltype(k)::value;
+        float v[16], s = 1.f, b = 0.f;
+        if constexpr (K != CK_F16 && K != CK_F32) {
+          s = half_bits(x.s, 0);
+          b = x.format == DC_FMT_M0_AFFINE ? half_bits(x.b, 0) : K == CK_I8 ? 0.f : -float((1 << (x.bits - 1)) - 1) * s;
+        }
+        values16<K>(x.r, x.shift, s, b, v);
         if (!x.live) return;
 #pragma unroll
         for (int q = 0; q < QB; ++q)

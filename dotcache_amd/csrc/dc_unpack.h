@@ -32,33 +32,75 @@ __host__ __device__ inline bool chunk16_geometry(const dc_page_geometry& g) {
   return g.head_dim % 16 == 0 && g.group_size % 16 == 0 && int64_t(g.page_capacity) * num_groups(g) * g.group_size < (1 << 28);
 }
 
-// Where a chunk's words, scale and bias sit in its blob, in bytes.  Every
-// field is linear in the token: add t times the step.
-struct Chunk16 {
-  uint32_t word, word_step;    // first raw word
-  uint32_t scale, scale_step;  // fp16 scale (M0, int8 rows)
-  uint32_t bias;               // fp16 bias (affine; same step as the scale)
-  int shift;                   // 3-bit codes: bit of channel 0 in the first word (0 or 16)
+// blob_layout in 32 bits, for geometries chunk16_geometry accepts (their
+// blobs stay below 2^30 bytes): a page's layout costs a few instructions.
+struct Blob32 {
+  uint32_t groups, words, scales_off, bias_off, total;
 };
 
-__device__ __forceinline__ Chunk16 chunk16_at(int32_t fmt, int32_t bits, const dc_page_geometry& geo, const BlobLayout& L,
-                                              int32_t c0) {
+__host__ __device__ inline Blob32 blob32(int32_t fmt, int32_t bits, const dc_page_geometry& g, uint32_t groups) {
+  const uint32_t C = g.page_capacity;
+  auto up16 = [](uint32_t x) { return (x + 15u) & ~15u; };
+  Blob32 L{};
+  L.groups = groups;
+  const bool m0 = is_m0(fmt);
+  L.words = m0 ? (uint32_t(g.group_size) * bits + 31) / 32 : 0;
+  const uint32_t es = fmt == DC_FMT_M3_F16 ? 2 : fmt == DC_FMT_M3_F32 ? 4 : 1;
+  L.scales_off = up16(m0 ? groups * C * L.words * 4 : C * uint32_t(g.head_dim) * es);
+  const uint32_t per = m0 ? up16(C * groups * 2) : fmt == DC_FMT_M3_I8 ? up16(C * 2) : 0;
+  L.bias_off = L.scales_off + per;
+  L.total = fmt == DC_FMT_M0_AFFINE ? L.bias_off + per : L.bias_off;
+  return L;
+}
+
+// A walk over a page's 16-channel chunks: where the current one's words,
+// scale and bias sit in the blob, in bytes.  Every offset is linear in the
+// token: add t times the step.  next() moves on without a division.
+struct Chunk16 {
+  uint32_t word_step, scale_step;  // per token
+  uint32_t base, bit;              // first word of the group (escapes: of the row), bit of the chunk from there
+  uint32_t scale, bias;
+  uint32_t chunk_bits, group_bits, group_step;  // (escapes: one group that never ends)
+
+  __device__ __forceinline__ uint32_t word() const { return base + (bit >> 5) * 4; }
+  __device__ __forceinline__ int shift() const { return int(bit & 31); }  // nonzero (16) for 3-bit codes only
+  __device__ __forceinline__ void next() {
+    bit += chunk_bits;
+    if (bit == group_bits) {
+      bit = 0;
+      base += group_step;
+      scale += 2;
+      bias += 2;
+    }
+  }
+};
+
+__device__ __forceinline__ Chunk16 chunk16_at(int32_t fmt, int32_t bits, const dc_page_geometry& geo, const Blob32& L,
+                                              uint32_t c0) {
   Chunk16 k{};
+  k.scale = L.scales_off;
+  k.bias = L.bias_off;
   if (is_m0(fmt)) {
-    const int32_t g = c0 / geo.group_size, bit = (c0 - g * geo.group_size) * bits;
-    const uint32_t row = L.words * 4;
-    k.word = (geo.layout == 0 ? uint32_t(g) * geo.page_capacity * row : g * row) + (bit >> 5) * 4;
+    const uint32_t gs = geo.group_size, row = L.words * 4;
+    k.chunk_bits = 16 * bits;
+    k.group_bits = gs * bits;
+    k.group_step = geo.layout == 0 ? uint32_t(geo.page_capacity) * row : row;
     k.word_step = geo.layout == 0 ? row : L.groups * row;
-    k.shift = bit & 31;
-    k.scale = uint32_t(L.scales_off) + 2 * g;
-    k.bias = uint32_t(L.bias_off) + 2 * g;
     k.scale_step = 2 * L.groups;
+    if (c0 != 0) {
+      const uint32_t g = c0 / gs;
+      k.bit = (c0 - g * gs) * bits;
+      k.base = g * k.group_step;
+      k.scale += 2 * g;
+      k.bias += 2 * g;
+    }
     return k;
   }
   const uint32_t es = fmt == DC_FMT_M3_F16 ? 2 : fmt == DC_FMT_M3_F32 ? 4 : 1;
-  k.word = c0 * es;
+  k.chunk_bits = 128 * es;
+  k.group_bits = ~0u;
+  k.bit = c0 * 8 * es;
   k.word_step = geo.head_dim * es;
-  k.scale = uint32_t(L.scales_off);
   k.scale_step = 2;
   return k;
 }
@@ -168,6 +210,75 @@ __device__ __forceinline__ void for_chunk_kind(int kind, F&& fn) {
     case CK_F32: fn(std::integral_constant<int, CK_F32>{}); break;
     default: break;
   }
+}
+
+// s0[n] + s1[n]: dot products of this lane's row (token t of the page d
+// describes) with the four queries of each register block n < NB, over hd
+// channels.  get_q(c0, n) is block n's query register of channels c0 .. c0 +
+// 15 (lane (b, r): channel c0 + b of its query r).  Two chunks in flight.
+template <int NB, typename GetQ>
+__device__ __forceinline__ void score_row(const dc_page_desc& d, const dc_page_geometry& geo, const Blob32& L,
+                                          const uint8_t* blob, uint32_t t, GetQ&& get_q, f32x4v (&s0)[NB],
+                                          f32x4v (&s1)[NB]) {
+  const int32_t hd = geo.head_dim;
+  // (a chunk holds what its loads return; conversions wait until it is used,
+  // or every load would be waited for where it was issued)
+  struct Chunk {
+    uint32_t r[16];
+    uint16_t s, b;
+    float q[NB];
+    int shift;
+  };
+  const float zp = -float((1 << (d.bits - 1)) - 1);
+  const bool affine = d.format == DC_FMT_M0_AFFINE;
+  Chunk16 ck = chunk16_at(d.format, d.bits, geo, L, 0);
+  const uint8_t* row = blob + t * ck.word_step;
+  const uint8_t* scales = blob + t * ck.scale_step;
+  for_chunk_kind(chunk_kind(d.format, d.bits), [&](auto kind) __attribute__((always_inline)) {
+    constexpr int K = decltype(kind)::value;
+    constexpr int D = K == CK_F32 ? 2 : 4;  // chunks in flight
+    auto load = [&](int32_t c0, Chunk& x) __attribute__((always_inline)) {
+      load_chunk16(K, row + ck.word(), x.r);
+      x.shift = ck.shift();
+      if constexpr (K != CK_F16 && K != CK_F32) {
+        x.s = *reinterpret_cast<const uint16_t*>(scales + ck.scale);
+        // (no bias: the scale again, unused)
+        x.b = *reinterpret_cast<const uint16_t*>(scales + (affine ? ck.bias : ck.scale));
+      }
+#pragma unroll
+      for (int n = 0; n < NB; ++n) x.q[n] = get_q(c0, n);
+      ck.next();
+    };
+    auto dot = [&](const Chunk& x) __attribute__((always_inline)) {
+      float v[16], s = 1.f, b = 0.f;
+      if constexpr (K != CK_F16 && K != CK_F32) {
+        s = half_bits(x.s, 0);
+        b = affine ? half_bits(x.b, 0) : K == CK_I8 ? 0.f : zp * s;
+      }
+      values16<K>(x.r, x.shift, s, b, v);
+#pragma unroll
+      for (int n = 0; n < NB; ++n) dot16(x.q[n], v, s0[n], s1[n]);
+    };
+    // whole rounds of D chunks without a branch, then the rest
+    Chunk X[D];
+    const int32_t n_chunks = hd / 16, whole = n_chunks / D * D;
+    if (whole > 0) {
+#pragma unroll
+      for (int j = 0; j < D; ++j) load(16 * j, X[j]);
+      for (int32_t c = D; c < whole; c += D)
+#pragma unroll
+        for (int j = 0; j < D; ++j) {
+          dot(X[j]);
+          load(16 * (c + j), X[j]);
+        }
+#pragma unroll
+      for (int j = 0; j < D; ++j) dot(X[j]);
+    }
+    for (int32_t c = whole; c < n_chunks; ++c) {
+      load(16 * c, X[0]);
+      dot(X[0]);
+    }
+  });
 }
 
 }  // namespace dc

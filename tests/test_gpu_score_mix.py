@@ -50,6 +50,41 @@ def test_grouped_logits_weights_and_output(fmt, hd, gs, tpp, Q, lens, layout):
         np.testing.assert_allclose(out[g], want[2], atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("kfmt,vfmt", [(FORMATS[i], FORMATS[(3 * i + 1) % len(FORMATS)]) for i in range(len(FORMATS))]
+                         + [(dict(bits=4), dict(mode="M3", escape_dtype="int8"))],
+                         ids=lambda f: "-".join(str(v) for v in f.values()))
+@pytest.mark.parametrize("hd,gs,vgs,tpp,Q,layout", [
+    (128, 32, 32, 64, 4, "group_major"),
+    (96, 32, 64, 96, 2, "group_major"),
+    (64, 16, 16, 32, 5, "token_major"),
+    (256, 64, 32, 256, 16, "group_major"),
+    (80, 16, 48, 100, 9, "group_major"),
+    (160, 32, 32, 64, 1, "token_major"),
+])
+def test_tile_decode_matches_oracle(kfmt, vfmt, hd, gs, vgs, tpp, Q, layout):
+    """The tile decode over the formats the matrix kernel does not take: token
+    counts of one unit, a partial unit, and several units per wave; one item
+    per group and items of two pages that split a group."""
+    from dotcache_amd.backends import decode_grouped_multiquery_step_prepared_hip_tensor_output_only as fused
+    from dotcache_amd.decode import set_decode_path
+
+    print(f"tiles {kfmt} {vfmt} hd {hd} gs {gs}/{vgs} page {tpp} Q {Q} {layout}", flush=True)
+    rng = np.random.default_rng(hd + tpp + Q)
+    lens = [1, 64, tpp + 17, 5 * tpp - 3]
+    q = (rng.normal(size=(len(lens), Q, hd)) / np.sqrt(hd)).astype(np.float32)
+    okp, kp = _groups(rng, hd, gs, kfmt, lens, tpp, "K", layout)
+    ovp, vp = _groups(rng, hd, vgs, vfmt, lens, tpp, "V", layout)
+    want = O.decode_grouped(q, okp, ovp)
+    set_decode_path("generic")
+    try:
+        for pps in (None, 2, 100):
+            got = fused(list(q), kp, vp, pages_per_split=pps).cpu().numpy()
+            # fp32 products and sums on both sides, |out| < 60
+            assert np.max(np.abs(got - want)) < 1e-4, f"pages per split {pps}"
+    finally:
+        set_decode_path("auto")
+
+
 def test_mix_keeps_infinities_of_valid_rows_only():
     """An infinite value row makes its channels infinite, not NaN, also as a
     page's last token."""
