@@ -16,8 +16,7 @@ every appended token.  Here a block id owns device pages directly:
 
 ``write_slots`` takes rows with a vLLM-style slot mapping (``block_id *
 block_size + offset``), and ``decode_block_tables`` decodes a batch of
-sequences given by block tables and context lengths in one launch: the
-page tables are gathered from the block map on the device.  The
+sequences given by block tables and context lengths in one launch.  The
 reference's single-sequence interface (``sync_layer_blocks``,
 ``append_step``, ``append_tokens_torch``, ``decode_layer``,
 ``block_entry``) is built on these two.
@@ -102,8 +101,10 @@ class DeviceVllmPagedKVCache:
         self._fill = [np.zeros(n, dtype=np.int32) for _ in range(L)]
         self._final = [np.zeros(n, dtype=bool) for _ in range(L)]
         self._start = [np.full(n, -1, dtype=np.int64) for _ in range(L)]
-        self._rows = [dict() for _ in range(L)]     # live block id -> fp32 rows [2, H, P, hd] on the device
-        self._dev_map = [None] * L                   # device copies of the K / V maps, rebuilt when they change
+        # fp32 rows of the live blocks, [slots, 2, H, P, hd] on the device; live block id -> slot
+        self._row_store = torch.empty((0, 2, H, P, hd), dtype=torch.float32, device=self.device)
+        self._row_slots = [dict() for _ in range(L)]
+        self._free_slots: list[int] = []
         # the single-sequence view of the reference interface: block ids in token order, cached length
         self._seq_blocks = [[] for _ in range(L)]
         self._seq_len = np.zeros(L, dtype=np.int64)
@@ -122,10 +123,13 @@ class DeviceVllmPagedKVCache:
         return lid
 
     def _as_rows(self, x, name: str):
-        """``x [n, H, hd]`` as fp32 on the device."""
+        """``x [n, H, hd]`` on the device in fp32, fp16 or bf16 (the encoder
+        reads each exactly as fp32); other types become fp32."""
         torch = _torch()
         t = x if isinstance(x, torch.Tensor) else torch.from_numpy(np.ascontiguousarray(np.asarray(x, dtype=np.float32)))
-        t = t.to(device=self.device, dtype=torch.float32)
+        t = t.to(device=self.device)
+        if t.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+            t = t.float()
         if t.dim() != 3 or t.shape[1] != self.num_key_value_heads or t.shape[2] != self.config.head_dim:
             raise ValueError(f"{name} must have shape [tokens, {self.num_key_value_heads}, {self.config.head_dim}]")
         return t
@@ -143,18 +147,42 @@ class DeviceVllmPagedKVCache:
         self._final[lid] = np.concatenate([self._final[lid], np.zeros(m - n, dtype=bool)])
         self._start[lid] = np.concatenate([self._start[lid], np.full(m - n, -1, dtype=np.int64)])
 
-    def _release(self, lid: int, block_id: int) -> None:
+    def _release(self, lid: int, blocks) -> None:
+        blocks = np.atleast_1d(np.asarray(blocks, dtype=np.int64))
         for kind in ("K", "V"):
-            ids = self._map[kind][lid][block_id]
-            live = ids[ids >= 0]
-            if len(live):
-                self._pools[kind].free(live)
-            ids[:] = -1
-        self._fill[lid][block_id] = 0
-        self._final[lid][block_id] = False
-        self._start[lid][block_id] = -1
-        self._rows[lid].pop(block_id, None)
-        self._dev_map[lid] = None
+            ids = self._map[kind][lid][blocks]
+            self._pools[kind].free(ids[ids >= 0])
+            self._map[kind][lid][blocks] = -1
+        self._fill[lid][blocks] = 0
+        self._final[lid][blocks] = False
+        self._start[lid][blocks] = -1
+        for blk in blocks.tolist():
+            if blk in self._row_slots[lid]:
+                self._free_slots.append(self._row_slots[lid].pop(blk))
+
+    def _take_slots(self, lid: int, blocks: list[int]) -> None:
+        """An fp32 row slot for every block (the store doubles when none is free)."""
+        torch = _torch()
+        short = len(blocks) - len(self._free_slots)
+        if short > 0:
+            n = int(self._row_store.shape[0])
+            m = max(2 * n, n + short)
+            grown = torch.empty((m, *self._row_store.shape[1:]), dtype=torch.float32, device=self.device)
+            grown[:n].copy_(self._row_store)
+            self._row_store = grown
+            self._free_slots.extend(range(m - 1, n - 1, -1))
+        for blk in blocks:
+            self._row_slots[lid][blk] = self._free_slots.pop()
+
+    def _allocate_final(self, kind: str, lid: int, n: int) -> np.ndarray:
+        """Page ids ``[n, H]`` in the layer's modes."""
+        H, P = self.num_key_value_heads, self.block_size
+        fmts = [self._page_format(kind, lid, h) for h in range(H)]
+        ids = np.empty((n, H), dtype=np.int32)
+        for f in set(fmts):
+            heads = [h for h in range(H) if fmts[h] == f]
+            ids[:, heads] = self._pools[kind].allocate(*f, n * len(heads), tokens=P).reshape(n, len(heads))
+        return ids
 
     # ---- the serving interface -------------------------------------------------
     def write_slots(self, layer_id: int, key_rows, value_rows, slot_mapping, *, token_start: int | None = None) -> None:
@@ -175,60 +203,107 @@ class DeviceVllmPagedKVCache:
             raise ValueError("slot_mapping needs one slot per row")
         if np.any(slots < 0):
             raise ValueError("slots must be non-negative")
-        P, H, hd = self.block_size, self.num_key_value_heads, self.config.head_dim
-        i = 0
+        P = self.block_size
         n = slots.shape[0]
-        while i < n:  # runs of consecutive slots of one block
-            blk, off = int(slots[i] // P), int(slots[i] % P)
-            j = i + 1
-            while j < n and slots[j] == slots[j - 1] + 1 and slots[j] // P == blk:
-                j += 1
+        if n == 0:
+            return
+        if keys.dtype != values.dtype:
+            keys, values = keys.float(), values.float()
+        # runs of consecutive slots of one block
+        blocks, offs = slots // P, slots % P
+        ends = np.append(np.flatnonzero((np.diff(slots) != 1) | (np.diff(blocks) != 0)) + 1, n).tolist()
+        runs: list[tuple[int, int, int, int]] = []  # (block, offset, first row, end row), checked
+        fills: dict[int, int] = {}                  # fill of the blocks of `runs` once they are written
+        restart: list[int] = []                     # blocks reused from their first slot
+        i, error = 0, None
+        for j in ends:
+            blk, off = int(blocks[i]), int(offs[i])
             self._grow(lid, blk)
-            if off == 0 and self._fill[lid][blk] > 0:
-                self._release(lid, blk)  # a block id reused from its first slot
-            if off != self._fill[lid][blk]:
-                raise ValueError(f"block {blk} holds {int(self._fill[lid][blk])} tokens; slot offset {off} is out of order")
-            self._write_run(lid, blk, off, keys[i:j], values[i:j], None if token_start is None else int(token_start) + i)
+            if off == 0 and blk in fills:  # written and reused in one call: the rows so far land first
+                self._write_runs(lid, runs, restart, keys, values, offs, token_start)
+                runs, fills, restart = [], {}, []
+            fill = fills.get(blk, int(self._fill[lid][blk]))
+            if off == 0 and fill > 0:
+                restart.append(blk)
+                fill = 0
+            if off != fill:
+                error = ValueError(f"block {blk} holds {fill} tokens; slot offset {off} is out of order")
+                break
+            runs.append((blk, off, i, j))
+            fills[blk] = off + j - i
             i = j
+        self._write_runs(lid, runs, restart, keys, values, offs, token_start)
+        if error is not None:
+            raise error
 
-    def _write_run(self, lid: int, blk: int, off: int, keys, values, start: int | None) -> None:
+    def _write_runs(self, lid: int, runs, restart, keys, values, offs: np.ndarray, token_start: int | None) -> None:
+        """Rows of checked runs in one launch (two when blocks fill up).  A
+        block written whole is encoded straight into its final pages; rows
+        of a live block go to its escape pages and, in fp32, to its row
+        slot; rows that fill a live block only to its row slot, from which
+        the block is then encoded."""
+        if restart:
+            self._release(lid, restart)
+        if not runs:
+            return
+        P, H, hd = self.block_size, self.num_key_value_heads, self.config.head_dim
+        blk = np.asarray([r[0] for r in runs], dtype=np.int64)
+        off, first, end = (np.asarray([r[k] for r in runs], dtype=np.int64) for k in (1, 2, 3))
+        full = off + end - first == P
+        whole = full & (off == 0)
+        fresh = (off == 0) & ~whole
+        self._start[lid][blk[off == 0]] = -1 if token_start is None else int(token_start) + first[off == 0]
+        for kind in ("K", "V"):
+            pool, table = self._pools[kind], self._map[kind][lid]
+            if whole.any():
+                table[blk[whole]] = self._allocate_final(kind, lid, int(whole.sum()))
+            if fresh.any():
+                table[blk[fresh]] = pool.allocate(*self._live_fmt[kind], int(fresh.sum()) * H, tokens=0).reshape(-1, H)
+            live = ~full
+            if live.any():
+                pool.set_tokens(table[blk[live]].ravel(), np.repeat((off + end - first)[live], H))
+        self._take_slots(lid, blk[fresh].tolist())
+        self._fill[lid][blk] = off + end - first
+        self._final[lid][blk[whole]] = True
+
+        # row (token i, head h): page ids (-1 where only the row slot takes it), slot, row of the store
+        a, z = int(first[0]), int(end[-1])
+        run = np.repeat(np.arange(len(runs)), end - first)
+        slot = offs[a:z]
+        heads = np.arange(H)
+        ids = [np.where((full & ~whole)[run][:, None], -1, self._map[kind][lid][blk][run]) for kind in ("K", "V")]
+        rows = self._row_slots[lid]
+        stored = np.asarray([-1 if w else rows[b] for b, w in zip(blk.tolist(), whole.tolist())], dtype=np.int64)[run]
+        keep = np.where(stored[:, None] < 0, -1, (stored[:, None] * 2 * H + heads) * P + slot[:, None])
+        slots = np.repeat(slot, H)
+        flat = self._row_store.view(-1, hd)
+        kept = None
+        if not whole.all():
+            kept = (flat[: flat.shape[0] - H * P], flat[H * P:], keep.ravel())
+        self.k_pool.encode_rows_with(self.v_pool, keys[a:z].reshape(-1, hd), values[a:z].reshape(-1, hd), ids[0].ravel(),
+                                     slots, ids[1].ravel(), slots, keep=kept)
+        done = blk[full & ~whole]
+        if done.size:
+            self._finalise(lid, done)
+
+    def _finalise(self, lid: int, blocks: np.ndarray) -> None:
+        """Encode full live blocks from their fp32 rows and release their
+        escape pages and row slots."""
         torch = _torch()
         P, H, hd = self.block_size, self.num_key_value_heads, self.config.head_dim
-        m = int(keys.shape[0])
-        if self._final[lid][blk]:
-            raise ValueError(f"block {blk} is full")
-        if blk not in self._rows[lid]:
-            self._rows[lid][blk] = torch.zeros((2, H, P, hd), dtype=torch.float32, device=self.device)
-            for kind in ("K", "V"):
-                self._map[kind][lid][blk] = self._pools[kind].allocate(*self._live_fmt[kind], H, tokens=0)
-            self._dev_map[lid] = None
-        if off == 0:
-            self._start[lid][blk] = -1 if start is None else start
-        rows = self._rows[lid][blk]
-        for k, (kind, x) in enumerate((("K", keys), ("V", values))):
-            xt = x.transpose(0, 1)  # [H, m, hd]
-            rows[k, :, off:off + m].copy_(xt)
-            ids = self._map[kind][lid][blk]
-            self._pools[kind].encode_rows(xt.reshape(H * m, hd), np.repeat(ids, m), np.tile(np.arange(off, off + m), H))
-            self._pools[kind].set_tokens(ids, off + m)
-        self._fill[lid][blk] = off + m
-        if off + m == P:
-            self._finalise(lid, blk)
-
-    def _finalise(self, lid: int, blk: int) -> None:
-        P, H, hd = self.block_size, self.num_key_value_heads, self.config.head_dim
-        rows = self._rows[lid].pop(blk)
-        for k, kind in enumerate(("K", "V")):
-            pool = self._pools[kind]
-            old = self._map[kind][lid][blk].copy()
-            new = np.empty(H, dtype=np.int32)
-            for h in range(H):
-                new[h] = pool.allocate(*self._page_format(kind, lid, h), 1, tokens=P)[0]
-            pool.encode_rows(rows[k].reshape(H * P, hd), np.repeat(new, P), np.tile(np.arange(P), H))
-            pool.free(old)
-            self._map[kind][lid][blk] = new
-        self._final[lid][blk] = True
-        self._dev_map[lid] = None
+        n = len(blocks)
+        at = [self._row_slots[lid].pop(b) for b in blocks.tolist()]
+        rows = self._row_store[at[0]][:, None] if n == 1 else self._row_store[torch.as_tensor(at, device=self.device)].transpose(0, 1)
+        new = {}
+        for kind in ("K", "V"):
+            old = self._map[kind][lid][blocks]
+            new[kind] = self._allocate_final(kind, lid, n)
+            self._pools[kind].free(old)
+            self._map[kind][lid][blocks] = new[kind]
+        tables = torch.from_numpy(np.stack([new["K"], new["V"]]).reshape(2, n * H, 1).astype(np.int32)).to(self.device)
+        self.k_pool.encode_streams_with(self.v_pool, rows[0].reshape(n * H, P, hd), rows[1].reshape(n * H, P, hd), tables)
+        self._free_slots.extend(at)
+        self._final[lid][blocks] = True
 
     def decode_block_tables(self, layer_id: int, queries, block_tables, context_lens, q_head_to_kv_head=None, *,
                             query_scale: float = 1.0):
@@ -258,30 +333,30 @@ class DeviceVllmPagedKVCache:
             raise ValueError("a context length needs more blocks than its block-table row holds")
         bt_host = bt.detach().cpu().numpy().astype(np.int64)
         nmap = self._fill[lid].shape[0]
-        for b in range(B):
-            used = bt_host[b, : n_blocks[b]]
-            if np.any(used < 0) or np.any(used >= nmap) or np.any(self._map["K"][lid][np.clip(used, 0, nmap - 1), 0] < 0):
+        at = np.clip(bt_host, 0, nmap - 1)
+        used = np.arange(bt_host.shape[1])[None, :] < n_blocks[:, None]
+        unknown = (used & ((bt_host < 0) | (bt_host >= nmap) | (self._map["K"][lid][at, 0] < 0))).any(axis=1)
+        held = np.where(used, self._fill[lid][at], 0).sum(axis=1)
+        wrong = np.flatnonzero(unknown | (held != lens))
+        if wrong.size:
+            b = int(wrong[0])
+            if unknown[b]:
                 raise ValueError(f"sequence {b} names a block with no pages in layer {lid}")
-            if int(self._fill[lid][used].sum()) != int(lens[b]):
-                raise ValueError(f"sequence {b}: its blocks hold {int(self._fill[lid][used].sum())} tokens, context_lens says {int(lens[b])}")
-        if self._dev_map[lid] is None:
-            self._dev_map[lid] = tuple(torch.from_numpy(self._map[kind][lid].astype(np.int32)).to(self.device) for kind in ("K", "V"))
-        idx = torch.from_numpy(np.clip(bt_host, 0, nmap - 1)).to(self.device)
-        k_table = self._dev_map[lid][0][idx].permute(0, 2, 1).contiguous()  # [B, H, W] page ids
-        v_table = self._dev_map[lid][1][idx].permute(0, 2, 1).contiguous()
+            raise ValueError(f"sequence {b}: its blocks hold {int(held[b])} tokens, context_lens says {int(lens[b])}")
+        # [B, H, W] page ids, keys and values
+        kt, vt = (self._map[kind][lid][at].transpose(0, 2, 1) for kind in ("K", "V"))
+        k_table, v_table = torch.from_numpy(np.ascontiguousarray(np.stack([kt, vt]))).to(self.device)
         qmap = self.default_q_head_to_kv_head if q_head_to_kv_head is None else np.asarray(q_head_to_kv_head, dtype=np.int64)
         if qmap.shape != (Hq,) or np.any(qmap < 0) or np.any(qmap >= H) or np.any(np.bincount(qmap, minlength=H) != Hq // H):
             raise ValueError("q_head_to_kv_head must give every KV head the same number of query heads")
         order = np.argsort(qmap, kind="stable")
         contiguous = np.array_equal(order, np.arange(Hq))
-        order_t = torch.from_numpy(order).to(self.device)
+        order_t = None if contiguous else torch.from_numpy(order).to(self.device)
         qg = (q if contiguous else q[:, order_t]).reshape(B, H, Hq // H, hd)
         seq_pages = n_blocks.astype(np.int32)
-        last_tokens = np.asarray([self._fill[lid][bt_host[b, n_blocks[b] - 1]] for b in range(B)], dtype=np.int32)
+        last_tokens = self._fill[lid][bt_host[np.arange(B), n_blocks - 1]]
         # (a sequence's live block is an fp16 page: the split-K merge attends
         # it, and the decode launch takes the instance of the full blocks)
-        kt = self._map["K"][lid][np.clip(bt_host, 0, nmap - 1)].transpose(0, 2, 1)
-        vt = self._map["V"][lid][np.clip(bt_host, 0, nmap - 1)].transpose(0, 2, 1)
         plan, masks = plan_decode(self.k_pool, self.v_pool, kt, vt, seq_pages, Hq // H, device=self.device,
                                   last_page_tokens=last_tokens)
         need = workspace_bytes(plan, Hq // H, hd)
@@ -433,8 +508,7 @@ class DeviceVllmPagedKVCache:
 
     def clear_layer(self, layer_id: int) -> None:
         lid = self._check_layer(layer_id)
-        for blk in np.flatnonzero((self._map["K"][lid][:, 0] >= 0) | (self._fill[lid] > 0)).tolist():
-            self._release(lid, blk)
+        self._release(lid, np.flatnonzero((self._map["K"][lid][:, 0] >= 0) | (self._fill[lid] > 0)))
         self._seq_blocks[lid] = []
         self._seq_len[lid] = 0
 

@@ -138,10 +138,13 @@ class DevicePagedKVCache:
 
     # ---- input normalisation ------------------------------------------------
     def _rows(self, x, *, tokens: int | None, name: str):
-        """``x`` as fp32 device ``[B, H, T, hd]``."""
+        """``x`` as device ``[B, H, T, hd]`` rows in fp32, fp16 or bf16 (the
+        encoder reads each exactly as fp32); other types become fp32."""
         torch = _torch()
         t = x if isinstance(x, torch.Tensor) else torch.from_numpy(np.ascontiguousarray(np.asarray(x, dtype=np.float32)))
-        t = t.to(device=self.device, dtype=torch.float32)
+        t = t.to(device=self.device)
+        if t.dtype not in (torch.float32, torch.float16, torch.bfloat16):
+            t = t.float()
         if t.dim() == 3 and self.batch_size == 1:
             t = t.unsqueeze(0)
         B, H, hd = self.batch_size, self.num_key_value_heads, self.config.head_dim
@@ -158,56 +161,63 @@ class DevicePagedKVCache:
         return lid
 
     # ---- writes ------------------------------------------------------------
-    def _encode(self, kind: str, rows, page_ids: np.ndarray, slots: np.ndarray) -> None:
-        if len(page_ids):
-            self._pool(kind).encode_rows(rows, page_ids.astype(np.int32), slots.astype(np.int32))
+    @staticmethod
+    def _one_dtype(keys, values):
+        return (keys, values) if keys.dtype == values.dtype else (keys.float(), values.float())
 
-    def _finalise_pages(self, kind: str, layer_id: int, rows, token_stream: np.ndarray, token_starts: np.ndarray,
-                        sequence_lengths: np.ndarray) -> None:
-        """Encode full pages: ``rows [n_pages * P, hd]`` fp32, page i of
-        stream ``token_stream[i]`` (index b * H + h) starting at absolute
-        token ``token_starts[i]`` of a context of ``sequence_lengths[i]``
-        tokens (the page-mode choice reads both)."""
+    def _new_pages(self, kind: str, layer_id: int, rows, token_starts: np.ndarray, sequence_lengths: np.ndarray) -> np.ndarray:
+        """Allocate full pages for every stream of a layer: ids ``[B * H, n]``,
+        page i of stream s starting at absolute token ``token_starts[s, i]``
+        of a context of ``sequence_lengths[s, i]`` tokens (the page-mode
+        choice reads both, and the page's fp32 rows, ``rows(s, i)``)."""
         P, H = self.config.tokens_per_page, self.num_key_value_heads
         pool = self._pool(kind)
-        n = len(token_stream)
-        specs = [self._page_spec(kind, layer_id, int(s) % H, int(t0), int(sl), rows[i * P:(i + 1) * P])
-                 for i, (s, t0, sl) in enumerate(zip(token_stream, token_starts, sequence_lengths))]
-        fmts = [page_format_of(sp["mode"], sp["scheme"], sp["bits"], sp["escape_dtype"]) for sp in specs]
-        ids = np.empty(n, dtype=np.int64)
-        for fmt_bits in set(fmts):
-            sel = [i for i in range(n) if fmts[i] == fmt_bits]
-            ids[sel] = pool.allocate(*fmt_bits, len(sel), tokens=P)
-        self._encode(kind, rows, np.repeat(ids, P), np.tile(np.arange(P), n))
-        for i, (pid, s) in enumerate(zip(ids.tolist(), token_stream.tolist())):
-            self._pages[kind][layer_id][s // H][s % H].append(pid)
-            pool.headers[pid] = make_header(self.config, specs[i], kind=kind, layer_id=layer_id, kv_head_id=s % H,
-                                            token_start=int(token_starts[i]), token_count=P)
+        S, n = token_starts.shape
+        if self.config.chooses_page_modes(kind):
+            specs = [[self._page_spec(kind, layer_id, s % H, int(token_starts[s, i]), int(sequence_lengths[s, i]), rows(s, i))
+                      for i in range(n)] for s in range(S)]
+        else:  # the mode depends on (kind, layer, head) only: one spec per stream
+            by_head = [self._page_spec(kind, layer_id, h, 0, 0, None) for h in range(H)]
+            specs = [[by_head[s % H]] for s in range(S)]
+        span = n // len(specs[0]) if n else 0  # pages per spec
+        fmts = [[page_format_of(sp["mode"], sp["scheme"], sp["bits"], sp["escape_dtype"]) for sp in row] for row in specs]
+        ids = np.empty((S, n), dtype=np.int64)
+        distinct = list({f: None for row in fmts for f in row}) if n else []
+        code = np.repeat([[distinct.index(f) for f in row] for row in fmts], span, axis=1) if n else ids
+        for k, fmt_bits in enumerate(distinct):
+            at = code == k
+            ids[at] = pool.allocate(*fmt_bits, int(at.sum()), tokens=P)
+        for s in range(S):
+            for k in range(len(specs[s]) if n else 0):
+                template = make_header(self.config, specs[s][k], kind=kind, layer_id=layer_id, kv_head_id=s % H,
+                                       token_start=0, token_count=P)
+                pool.headers.fill(ids[s, k * span:(k + 1) * span].tolist(), template,
+                                  token_starts[s, k * span:(k + 1) * span].tolist())
+            self._pages[kind][layer_id][s // H][s % H].extend(ids[s].tolist())
+        return ids
 
-    def _write_tail(self, kind: str, layer_id: int, rows, first_slot: int) -> None:
-        """Rows ``[B, H, n, hd]`` into tail slots ``first_slot ..`` of every
-        stream of the layer (fp32 copy and escape page)."""
-        B, H, n = int(rows.shape[0]), int(rows.shape[1]), int(rows.shape[2])
-        if n == 0:
-            return
+    def _tail_ids(self, kind: str, layer_id: int) -> np.ndarray:
+        """Tail page ids ``[B * H]`` of a layer, allocated on first use."""
         tp = self._tail_page[kind][layer_id]
-        pool = self._pool(kind)
         missing = np.argwhere(tp < 0)
         if len(missing):
-            ids = pool.allocate(*self._tail_fmt[kind], len(missing), tokens=0)
-            tp[missing[:, 0], missing[:, 1]] = ids
-        self._tail_rows[kind][layer_id, :, :, first_slot: first_slot + n].copy_(rows)
-        flat = rows.reshape(B * H * n, -1)
-        page_ids = np.repeat(tp.reshape(-1), n)
-        slots = np.tile(np.arange(first_slot, first_slot + n), B * H)
-        self._encode(kind, flat, page_ids, slots)
-        pool.set_tokens(tp.reshape(-1), first_slot + n)
+            tp[missing[:, 0], missing[:, 1]] = self._pool(kind).allocate(*self._tail_fmt[kind], len(missing), tokens=0)
+        return tp.reshape(-1)
+
+    def _upload_tables(self, k_ids: np.ndarray, v_ids: np.ndarray):
+        """Device int32 ``[2, streams, pages]`` page tables (keys, values)."""
+        return _torch().from_numpy(np.stack([k_ids, v_ids]).astype(np.int32)).to(self.device)
+
+    def _tails(self, layer_id: int) -> tuple:
+        """The layer's fp32 tail rows ``[B * H * P, hd]``, keys and values."""
+        return tuple(self._tail_rows[kind][layer_id].view(-1, self.config.head_dim) for kind in ("K", "V"))
 
     # ---- the reference's entry points ---------------------------------------
     def ingest_prefill_cache(self, layer_id: int, layer_k, layer_v, *, context_length: int | None = None) -> None:
         """Store a prefill's K/V ``[B, H, T, hd]`` for layer ``layer_id``:
         full pages are encoded on the device, the remaining ``T % P`` rows
-        become the tail (reference ``model_kv_cache.py:3609-3691``)."""
+        become the tail, all in one launch (reference
+        ``model_kv_cache.py:3609-3691``)."""
         lid = self._check_layer(layer_id)
         keys = self._rows(layer_k, tokens=None, name="layer_k")
         values = self._rows(layer_v, tokens=int(keys.shape[2]), name="layer_v")
@@ -216,20 +226,25 @@ class DevicePagedKVCache:
         if ctx < T:
             raise ValueError("context_length must be at least the stored prefill cache length")
         self.clear_layer(lid)
+        keys, values = self._one_dtype(keys, values)
         B, H, P, hd = self.batch_size, self.num_key_value_heads, self.config.tokens_per_page, self.config.head_dim
-        full = (T // P) * P
-        if full:
-            # page-major rows: stream (b, h), page i, slot j; page i starts at
-            # absolute token ctx - T + i P of a ctx-token context
-            streams = np.repeat(np.arange(B * H), full // P)
-            starts = np.tile((ctx - T) + P * np.arange(full // P), B * H)
-            for kind, x in (("K", keys), ("V", values)):
-                self._finalise_pages(kind, lid, x[:, :, :full].reshape(B * H * full, hd), streams, starts,
-                                     np.full(len(streams), ctx))
+        n = T // P
+        # stream (b, h), page i: tokens from ctx - T + i P of a ctx-token context
+        starts = np.broadcast_to((ctx - T) + P * np.arange(n), (B * H, n))
+        ids = {}
         for kind, x in (("K", keys), ("V", values)):
-            self._write_tail(kind, lid, x[:, :, full:], 0)
+            page_rows = lambda s, i, x=x: x[s // H, s % H, i * P:(i + 1) * P].float()  # noqa: E731
+            ids[kind] = self._new_pages(kind, lid, page_rows, starts, np.full((B * H, n), ctx))
+            if T > n * P:
+                tail = self._tail_ids(kind, lid)
+                self._pool(kind).set_tokens(tail, T - n * P)
+                ids[kind] = np.concatenate([ids[kind], tail[:, None]], axis=1)
         self._seq_len[lid, :] = ctx
-        self._tail_start[lid, :] = ctx - T + full
+        self._tail_start[lid, :] = ctx - T + n * P
+        if T:
+            tables = self._upload_tables(ids["K"], ids["V"])
+            self.k_pool.encode_streams_with(self.v_pool, keys.reshape(B * H, T, hd), values.reshape(B * H, T, hd), tables,
+                                            keep=self._tails(lid), keep_from=n * P)
         self._tables[lid] = None
 
     def append_step(self, layer_id: int, key_step, value_step, token_index: int) -> None:
@@ -242,27 +257,41 @@ class DevicePagedKVCache:
         values = self._rows(value_step, tokens=int(keys.shape[2]), name="value_step")
         if np.any(self._seq_len[lid] != int(token_index)):
             raise ValueError(f"layer {lid} expected token_index {int(self._seq_len[lid, 0])}, received {token_index}")
+        keys, values = self._one_dtype(keys, values)
         B, H, P, hd = self.batch_size, self.num_key_value_heads, self.config.tokens_per_page, self.config.head_dim
         n = int(keys.shape[2])
         done = 0
         while done < n:
             fill = int(self._seq_len[lid, 0] - self._tail_start[lid, 0])
             take = min(P - fill, n - done)
-            for kind, x in (("K", keys), ("V", values)):
-                self._write_tail(kind, lid, x[:, :, done: done + take], fill)
+            tails = [self._tail_ids(kind, lid) for kind in ("K", "V")]
+            for kind, tail in zip(("K", "V"), tails):
+                self._pool(kind).set_tokens(tail, fill + take)
+            # rows into the tail pages (exact) and the fp32 tail
+            self.k_pool.encode_streams_with(self.v_pool, keys[:, :, done: done + take].reshape(B * H, take, hd),
+                                            values[:, :, done: done + take].reshape(B * H, take, hd),
+                                            self._upload_tables(tails[0][:, None], tails[1][:, None]), first_slot=fill,
+                                            keep=self._tails(lid))
             done += take
             self._seq_len[lid, :] += take
             if fill + take == P:  # every stream's tail is full: encode it into a page
                 # the page's context is the whole step's (reference
                 # model_kv_cache.py:3887-3892 passes token_index + n)
-                streams = np.arange(B * H)
-                starts = np.repeat(self._tail_start[lid], H)
+                starts = np.repeat(self._tail_start[lid], H)[:, None]
+                ids = []
                 for kind in ("K", "V"):
-                    rows = self._tail_rows[kind][lid].reshape(B * H * P, hd)
-                    self._finalise_pages(kind, lid, rows, streams, starts, np.full(B * H, int(token_index) + n))
+                    rows = lambda s, i, kind=kind: self._tail_rows[kind][lid, s // H, s % H]  # noqa: E731
+                    ids.append(self._new_pages(kind, lid, rows, starts, np.full((B * H, 1), int(token_index) + n)))
                     self._pool(kind).set_tokens(self._tail_page[kind][lid].reshape(-1), 0)
+                self.k_pool.encode_streams_with(self.v_pool, *(t.view(B * H, P, hd) for t in self._tails(lid)),
+                                                self._upload_tables(*ids))
                 self._tail_start[lid, :] = self._seq_len[lid, :]
-            self._tables[lid] = None
+                self._tables[lid] = None
+            elif fill == 0:
+                self._tables[lid] = None  # the tail joins the tables
+            elif self._tables[lid] is not None:  # the same pages, a longer tail
+                k_table, v_table, counts, _ = self._tables[lid]
+                self._tables[lid] = (k_table, v_table, counts, np.full(B, fill + take, dtype=np.int32))
 
     def decode_layer(self, layer_id: int, query_step, q_head_to_kv_head=None, *, query_scale: float = 1.0):
         """Attention of ``query_step [B, Hq, hd]`` over layer ``layer_id``'s
@@ -323,19 +352,16 @@ class DevicePagedKVCache:
             has_tail = (self._seq_len[lid] - self._tail_start[lid]) > 0
             counts = np.array([len(self._pages["K"][lid][b][0]) + int(has_tail[b]) for b in range(B)], dtype=np.int32)
             stride = max(int(counts.max()), 1)
-            tabs, host = {}, {}
-            for kind in ("K", "V"):
-                t = np.zeros((B, H, stride), dtype=np.int32)
+            host = np.zeros((2, B, H, stride), dtype=np.int32)
+            for k, kind in enumerate(("K", "V")):
                 for b in range(B):
                     for h in range(H):
                         ids = self._pages[kind][lid][b][h] + ([int(self._tail_page[kind][lid, b, h])] if has_tail[b] else [])
-                        t[b, h, : len(ids)] = ids
-                tabs[kind] = torch.from_numpy(t).to(self.device)
-                host[kind] = t
-                if kind == "K":
-                    last = self.k_pool.tokens_of(t[np.arange(B), 0, np.maximum(counts - 1, 0)]).astype(np.int32)
-            self._tables[lid] = (tabs["K"], tabs["V"], counts, last)
-            self._host_tables[lid] = (host["K"], host["V"])
+                        host[k, b, h, : len(ids)] = ids
+            last = self.k_pool.tokens_of(host[0, np.arange(B), 0, np.maximum(counts - 1, 0)]).astype(np.int32)
+            k_table, v_table = torch.from_numpy(host).to(self.device)
+            self._tables[lid] = (k_table, v_table, counts, last)
+            self._host_tables[lid] = (host[0], host[1])
         return self._tables[lid]
 
     def clear_layer(self, layer_id: int) -> None:

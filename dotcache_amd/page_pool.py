@@ -22,7 +22,7 @@ from __future__ import annotations
 
 import ctypes as C
 from collections import deque
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 
 import numpy as np
 
@@ -30,6 +30,11 @@ from . import _lib
 from .types import EncodedPage, PageHeader, words_per_group
 
 DESC_DTYPE = np.dtype([("block", "<u4"), ("tokens", "<u2"), ("format", "u1"), ("bits", "u1")])
+
+# Pools of up to this many pages upload their whole descriptor table (8 bytes
+# a page) when some of it changed: one copy of at most 64 KiB costs the host
+# less than an index upload, a value upload and a scatter launch.
+WHOLE_TABLE_PAGES = 8192
 
 _SCHEME_FMT = {"affine": _lib.FMT_M0_AFFINE, "symmetric": _lib.FMT_M0_SYMMETRIC}
 _ESCAPE_FMT = {"float16": _lib.FMT_M3_F16, "float32": _lib.FMT_M3_F32, "int8": _lib.FMT_M3_I8}
@@ -96,6 +101,82 @@ class PoolGeometry:
         return _lib.geometry(self.head_dim, self.group_size, self.page_capacity, self.layout)
 
 
+class _PageHeaders(dict):
+    """Page id -> header.  ``fill`` registers the headers of a batch of pages
+    that differ in ``token_start`` only; each is made when it is first asked
+    for."""
+
+    def __init__(self):
+        super().__init__()
+        self._deferred: dict[int, tuple[PageHeader, int]] = {}
+
+    def discard(self, page_ids: list[int]) -> None:
+        """Drop these pages' headers, without making deferred ones."""
+        if self._deferred:
+            for pid in page_ids:
+                self._deferred.pop(pid, None)
+        if dict.__len__(self):
+            for pid in page_ids:
+                dict.pop(self, pid, None)
+
+    def fill(self, page_ids: list[int], template: PageHeader, token_starts: list[int]) -> None:
+        self.discard(page_ids)
+        self._deferred.update(zip(page_ids, ((template, t) for t in token_starts)))
+
+    def _make(self, pid):
+        template, start = self._deferred.pop(pid)
+        h = replace(template, token_start=start)
+        super().__setitem__(pid, h)
+        return h
+
+    def __setitem__(self, pid, header):
+        self._deferred.pop(pid, None)
+        super().__setitem__(pid, header)
+
+    def __missing__(self, pid):
+        if pid in self._deferred:
+            return self._make(pid)
+        raise KeyError(pid)
+
+    def get(self, pid, default=None):
+        return self._make(pid) if pid in self._deferred else super().get(pid, default)
+
+    def pop(self, pid, *default):
+        if pid in self._deferred:
+            template, start = self._deferred.pop(pid)
+            return replace(template, token_start=start)
+        return super().pop(pid, *default)
+
+    def __contains__(self, pid):
+        return pid in self._deferred or super().__contains__(pid)
+
+    def _all(self):
+        for pid in list(self._deferred):
+            self._make(pid)
+
+    def __iter__(self):
+        self._all()
+        return super().__iter__()
+
+    def keys(self):
+        self._all()
+        return super().keys()
+
+    def values(self):
+        self._all()
+        return super().values()
+
+    def items(self):
+        self._all()
+        return super().items()
+
+    def __len__(self):
+        return len(self._deferred) + super().__len__()
+
+    def __bool__(self):
+        return len(self) > 0
+
+
 class DevicePagePool:
     """Arena + descriptor table on one device.
 
@@ -126,8 +207,8 @@ class DevicePagePool:
         # bumped on every descriptor change: page records gathered at one
         # version are stale at any other
         self.desc_version = 0
-        self.headers: dict[int, PageHeader] = {}
-        self._blob_size: dict[int, int] = {}
+        self.headers: dict[int, PageHeader] = _PageHeaders()
+        self._blob_blocks = np.zeros(self._host_desc.shape[0], dtype=np.int64)  # 256-byte blocks of each live page's blob
         self._live = np.zeros(self._host_desc.shape[0], dtype=bool)
 
     # ---- bookkeeping -----------------------------------------------------
@@ -149,58 +230,76 @@ class DevicePagePool:
             new[:used].copy_(self.arena[:used])
         self.arena = new
 
-    def _new_id(self) -> int:
-        if self._free_ids:
-            return self._free_ids.popleft()
-        if self._n_pages == self._host_desc.shape[0]:
-            grown = np.zeros(2 * self._host_desc.shape[0], dtype=DESC_DTYPE)
-            grown[: self._n_pages] = self._host_desc[: self._n_pages]
-            self._host_desc = grown
-            live = np.zeros(grown.shape[0], dtype=bool)
-            live[: self._n_pages] = self._live[: self._n_pages]
-            self._live = live
-        pid = self._n_pages
-        self._n_pages += 1
-        return pid
+    def _new_ids(self, count: int) -> np.ndarray:
+        """``count`` page ids: freed ones first (oldest first), then new ones."""
+        reuse = min(count, len(self._free_ids))
+        old = [self._free_ids.popleft() for _ in range(reuse)]
+        end = self._n_pages + count - reuse
+        cap = self._host_desc.shape[0]
+        if end > cap:
+            while cap < end:
+                cap *= 2
+            for name in ("_host_desc", "_live", "_blob_blocks"):
+                a = getattr(self, name)
+                grown = np.zeros(cap, dtype=a.dtype)
+                grown[: self._n_pages] = a[: self._n_pages]
+                setattr(self, name, grown)
+        ids = np.asarray(old + list(range(self._n_pages, end)), dtype=np.int32)
+        self._n_pages = end
+        return ids
+
+    def _place(self, ids: np.ndarray, blocks, tokens, fmt: int, bits: int, nblk: int) -> None:
+        """Descriptors of new live pages ``ids`` of one format."""
+        d = self._host_desc
+        d["block"][ids], d["tokens"][ids], d["format"][ids], d["bits"][ids] = blocks, tokens, fmt, bits
+        self.format_mask |= _lib.format_bit(fmt, bits)
+        self._live[ids] = True
+        self._blob_blocks[ids] = nblk
+        self._dirty_ids.update(ids.tolist())
+        self.desc_version += 1
+
+    def _take_blocks(self, nblk: int, count: int) -> list[int]:
+        """Blob starts for ``count`` pages of ``nblk`` blocks: freed blobs of
+        that size first (the last freed first), then fresh contiguous ones."""
+        free = self._free.get(nblk, [])
+        reuse = min(count, len(free))
+        blocks = free[len(free) - reuse:][::-1]
+        self._ensure_arena(self._next_block + (count - reuse) * nblk)
+        if reuse:
+            del free[len(free) - reuse:]
+        start = self._next_block
+        self._next_block += (count - reuse) * nblk
+        return blocks + list(range(start, self._next_block, nblk))
 
     def allocate(self, fmt: int, bits: int, count: int = 1, *, tokens: int = 0) -> np.ndarray:
         """Allocate ``count`` page blobs of one format; returns int32 page ids.
         Fresh blobs are contiguous, so a batch upload is one copy."""
-        nbytes = self.blob_bytes(fmt, bits)
-        nblk = nbytes // 256
-        ids = np.empty(count, dtype=np.int32)
-        free = self._free.get(nblk, [])
-        fresh = max(0, count - len(free))
-        self._ensure_arena(self._next_block + fresh * nblk)
-        for i in range(count):
-            if free:
-                block = free.pop()
-            else:
-                block = self._next_block
-                self._next_block += nblk
-            pid = self._new_id()
-            self._host_desc[pid] = (block, tokens, fmt, bits)
-            self.format_mask |= _lib.format_bit(fmt, bits)
-            self._live[pid] = True
-            self._blob_size[pid] = nblk
-            ids[i] = pid
-        self._dirty_ids.update(ids.tolist())
-        self.desc_version += 1
+        nblk = self.blob_bytes(fmt, bits) // 256
+        blocks = self._take_blocks(nblk, count)
+        ids = self._new_ids(count)
+        if count:
+            self._place(ids, blocks, tokens, fmt, bits, nblk)
         return ids
 
     def free(self, page_ids) -> None:
-        for pid in np.atleast_1d(np.asarray(page_ids, dtype=np.int64)):
-            pid = int(pid)
-            if not self._live[pid]:
-                raise RuntimeError(f"page {pid} is not live")
-            self._live[pid] = False
-            nblk = self._blob_size.pop(pid)
-            self._free.setdefault(nblk, []).append(int(self._host_desc[pid]["block"]))
-            self._host_desc[pid] = (0, 0, 0, 0)
-            self.headers.pop(pid, None)
-            self._dirty_ids.add(pid)
-            self._free_ids.append(pid)
-            self.desc_version += 1
+        ids = np.atleast_1d(np.asarray(page_ids, dtype=np.int64)).ravel()
+        listed = ids.tolist()
+        if ids.size == 0:
+            return
+        dead = ids[~self._live[ids]]
+        if dead.size:
+            raise RuntimeError(f"page {int(dead[0])} is not live")
+        if len(set(listed)) != ids.size:
+            raise RuntimeError("a page is listed twice: it is not live once freed")
+        self._live[ids] = False
+        sizes, starts = self._blob_blocks[ids], self._host_desc["block"][ids]
+        for nblk in set(sizes.tolist()):
+            self._free.setdefault(nblk, []).extend(starts[sizes == nblk].tolist())
+        self._host_desc[ids] = np.zeros((), dtype=DESC_DTYPE)
+        self.headers.discard(listed)
+        self._dirty_ids.update(listed)
+        self._free_ids.extend(listed)
+        self.desc_version += 1
 
     def set_tokens(self, page_ids, tokens) -> None:
         ids = np.atleast_1d(np.asarray(page_ids, dtype=np.int64)).ravel()
@@ -208,11 +307,13 @@ class DevicePagePool:
         if np.any(tok < 0) or np.any(tok > self.geometry.page_capacity):
             raise ValueError("token count outside [0, page_capacity]")
         self._host_desc["tokens"][ids] = tok
-        for pid, t in zip(ids.tolist(), tok.tolist()):
-            h = self.headers.get(pid)
-            if h is not None:
-                h.token_count = int(t)
-        self._dirty_ids.update(ids.tolist())
+        listed = ids.tolist()
+        if self.headers:
+            for pid, t in zip(listed, tok.tolist()):
+                h = self.headers.get(pid)
+                if h is not None:
+                    h.token_count = int(t)
+        self._dirty_ids.update(listed)
         self.desc_version += 1
 
     def desc(self, page_id: int):
@@ -232,13 +333,14 @@ class DevicePagePool:
     def format_mask_of(self, page_ids) -> int:
         """``dc_pool.format_mask`` bits of the formats these pages hold (a
         subset of :attr:`format_mask`)."""
-        ids = np.unique(np.asarray(page_ids, dtype=np.int64).ravel())
+        ids = np.asarray(page_ids, dtype=np.int64).ravel()
         if ids.size == 0:
             return 0
-        d = self._host_desc[ids]
+        d = self._host_desc
+        seen = np.bincount(d["format"][ids].astype(np.int64) * 16 + d["bits"][ids])
         mask = 0
-        for fmt, bits in set(zip(d["format"].tolist(), d["bits"].tolist())):
-            mask |= _lib.format_bit(int(fmt), int(bits))
+        for code in np.flatnonzero(seen).tolist():
+            mask |= _lib.format_bit(code >> 4, code & 15)
         return mask
 
     def validate_ids(self, page_ids) -> None:
@@ -248,8 +350,8 @@ class DevicePagePool:
 
     def device_descs(self):
         """Device copy of the descriptor table, sized like the host table.
-        Changed descriptors are copied up by index; the whole table only
-        when the host table has outgrown the device copy."""
+        Changed descriptors are copied up by index; the whole table when it
+        is short or the host table has outgrown the device copy."""
         torch = _torch()
         cap = self._host_desc.shape[0]
         if self._dev_desc is None or self._dev_desc.numel() < cap:
@@ -257,9 +359,13 @@ class DevicePagePool:
             self._dev_desc = torch.from_numpy(raw).to(self.device, non_blocking=False)
             self._dirty_ids.clear()
         elif self._dirty_ids:
-            ids = np.fromiter(sorted(self._dirty_ids), dtype=np.int64, count=len(self._dirty_ids))
-            vals = torch.from_numpy(self._host_desc[ids].view(np.int64).copy()).to(self.device, non_blocking=False)
-            self._dev_desc[torch.from_numpy(ids).to(self.device)] = vals
+            if self._n_pages <= WHOLE_TABLE_PAGES:
+                raw = self._host_desc[: self._n_pages].view(np.int64).copy()
+                self._dev_desc[: self._n_pages].copy_(torch.from_numpy(raw))
+            else:
+                ids = np.fromiter(sorted(self._dirty_ids), dtype=np.int64, count=len(self._dirty_ids))
+                both = torch.from_numpy(np.stack([ids, self._host_desc[ids].view(np.int64)])).to(self.device)
+                self._dev_desc[both[0]] = both[1]
             self._dirty_ids.clear()
         return self._dev_desc
 
@@ -333,23 +439,14 @@ class DevicePagePool:
             src = torch.from_numpy(host)
             if self.device.type == "cuda":
                 src = src.pin_memory()
-            free = self._free.get(nblk, [])
-            n_old = min(len(free), len(idx))
-            blocks = [free.pop() for _ in range(n_old)]
+            n_old = min(len(self._free.get(nblk, [])), len(idx))
             start = self._next_block
-            self._ensure_arena(start + (len(idx) - n_old) * nblk)
-            blocks += [start + j * nblk for j in range(len(idx) - n_old)]
-            self._next_block = start + (len(idx) - n_old) * nblk
-            for i, block in zip(idx, blocks):
-                pid = self._new_id()
-                self._host_desc[pid] = (block, pages[i].header.token_count, fmt, bits)
-                self.format_mask |= _lib.format_bit(fmt, bits)
-                self._live[pid] = True
-                self._blob_size[pid] = nblk
-                self.headers[pid] = PageHeader.from_dict(pages[i].header.to_dict())
-                self._dirty_ids.add(pid)
-                self.desc_version += 1
-                ids[i] = pid
+            blocks = self._take_blocks(nblk, len(idx))
+            new = self._new_ids(len(idx))
+            self._place(new, blocks, [pages[i].header.token_count for i in idx], fmt, bits, nblk)
+            ids[idx] = new
+            for i, pid in zip(idx, new.tolist()):
+                self.headers[pid] = replace(pages[i].header)
             if n_old == 0:  # fresh contiguous blocks: one copy
                 self.arena[start * 256: start * 256 + host.size].copy_(src, non_blocking=False)
             else:  # one upload, then a scatter of 256-byte rows into the reused blobs
@@ -432,10 +529,13 @@ class DevicePagePool:
         _lib.check(st, "dc_encode_rows")
 
     def encode_rows_with(self, v_pool: "DevicePagePool", k_values, v_values, k_page_ids, k_slots, v_page_ids,
-                         v_slots) -> None:
+                         v_slots, *, keep=None) -> None:
         """Keys into this pool and values into ``v_pool`` in one launch
         (``dc_encode_rows_kv``): the per-step append of new tokens.  Both
-        value arrays are ``[n, head_dim]`` of one dtype and row stride."""
+        value arrays are ``[n, head_dim]`` of one dtype and row stride.
+        ``keep = (k_rows, v_rows, row)`` also stores row i unencoded at row
+        ``row[i]`` (-1: not) of two fp32 buffers ``[m, head_dim]``; a row
+        whose page id is -1 is only kept (``dc_encode_rows_kv_keep``)."""
         torch = _torch()
         hd = self.geometry.head_dim
         if v_pool.geometry.head_dim != hd:
@@ -446,14 +546,56 @@ class DevicePagePool:
             raise ValueError("key and value rows must have the same dtype")
         k_values, v_values = k_values.contiguous(), v_values.contiguous()
         n = k_values.shape[0]
-        ids = [torch.as_tensor(x, dtype=torch.int32, device=self.device).contiguous()
-               for x in (k_page_ids, k_slots, v_page_ids, v_slots)]
+        lists = [k_page_ids, k_slots, v_page_ids, v_slots] + ([keep[2]] if keep is not None else [])
+        if all(isinstance(x, np.ndarray) for x in lists):  # host lists: one upload
+            if any(x.size != n for x in lists):
+                raise ValueError("page_ids and slots must have one entry per row")
+            ids = list(torch.from_numpy(np.stack([x.reshape(-1).astype(np.int32) for x in lists])).to(self.device))
+        else:
+            ids = [torch.as_tensor(x, dtype=torch.int32, device=self.device).contiguous() for x in lists]
         if any(t.numel() != n for t in ids):
             raise ValueError("page_ids and slots must have one entry per row")
-        st = _lib.lib().dc_encode_rows_kv(
-            C.c_void_p(k_values.data_ptr()), C.c_void_p(v_values.data_ptr()), dtype_code(k_values), n, hd,
-            *(C.c_void_p(t.data_ptr()) for t in ids), self.c_pool(), v_pool.c_pool(), C.c_void_p(current_stream_ptr()))
+        args = (C.c_void_p(k_values.data_ptr()), C.c_void_p(v_values.data_ptr()), dtype_code(k_values), n, hd,
+                *(C.c_void_p(t.data_ptr()) for t in ids[:4]), self.c_pool(), v_pool.c_pool())
+        if keep is None:
+            st = _lib.lib().dc_encode_rows_kv(*args, C.c_void_p(current_stream_ptr()))
+        else:
+            for t in keep[:2]:
+                if t.dim() != 2 or t.shape != keep[0].shape or t.shape[1] != hd or t.dtype != torch.float32 or not t.is_contiguous():
+                    raise ValueError("kept rows must be two contiguous fp32 tensors [m, head_dim]")
+            st = _lib.lib().dc_encode_rows_kv_keep(*args, C.c_void_p(keep[0].data_ptr()), C.c_void_p(keep[1].data_ptr()),
+                                                   C.c_void_p(ids[4].data_ptr()), int(keep[0].shape[0]),
+                                                   C.c_void_p(current_stream_ptr()))
         _lib.check(st, "dc_encode_rows_kv")
+
+    def encode_streams_with(self, v_pool: "DevicePagePool", k_values, v_values, tables, *, first_slot: int = 0,
+                            keep=None, keep_from: int = 0) -> None:
+        """Keys ``[S, T, head_dim]`` of S token streams into this pool and
+        values into ``v_pool`` in one launch (``dc_encode_streams_kv``):
+        token t of stream s is token u = ``first_slot`` + t of its page-table
+        row and goes to slot u % capacity of page ``tables[kind, s, u //
+        capacity]`` (int32 device ``[2, S, pages]``, keys first).  ``keep``:
+        fp32 buffers ``[S * capacity, head_dim]`` (keys, values) that also
+        take tokens u >= ``keep_from`` unencoded, at row s * capacity + slot."""
+        torch = _torch()
+        hd, cap = self.geometry.head_dim, self.geometry.page_capacity
+        if (v_pool.geometry.head_dim, v_pool.geometry.page_capacity) != (hd, cap):
+            raise ValueError("key and value pools must share head_dim and page_capacity")
+        if k_values.dim() != 3 or k_values.shape[2] != hd or v_values.shape != k_values.shape or v_values.dtype != k_values.dtype:
+            raise ValueError("key and value rows must have one shape [streams, tokens, head_dim] and dtype")
+        S, T = int(k_values.shape[0]), int(k_values.shape[1])
+        if tables.dtype != torch.int32 or tables.dim() != 3 or tuple(tables.shape[:2]) != (2, S) or not tables.is_contiguous():
+            raise ValueError("tables must be contiguous int32 [2, streams, pages]")
+        for t in keep or ():
+            if tuple(t.shape) != (S * cap, hd) or t.dtype != torch.float32 or not t.is_contiguous():
+                raise ValueError("kept rows must be contiguous fp32 [streams * page_capacity, head_dim]")
+        k_values, v_values = k_values.contiguous(), v_values.contiguous()
+        st = _lib.lib().dc_encode_streams_kv(
+            C.c_void_p(k_values.data_ptr()), C.c_void_p(v_values.data_ptr()), dtype_code(k_values), S, T, hd,
+            C.c_void_p(tables[0].data_ptr()), C.c_void_p(tables[1].data_ptr()), int(tables.shape[2]), int(first_slot), cap,
+            self.c_pool(), v_pool.c_pool(), C.c_void_p(keep[0].data_ptr() if keep else 0),
+            C.c_void_p(keep[1].data_ptr() if keep else 0), int(keep_from), C.c_void_p(current_stream_ptr()))
+        _lib.check(st, "dc_encode_streams_kv")
 
     def read_bytes(self, page_ids) -> int:
         """Compressed bytes a reader fetches for these pages (valid tokens only)."""

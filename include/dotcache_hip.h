@@ -186,6 +186,30 @@ int dc_encode_rows_kv(const void* k_values, const void* v_values, int32_t values
                       const int32_t* v_row_page, const int32_t* v_row_slot, dc_pool k_pool, dc_pool v_pool,
                       dc_stream_t stream);
 
+/* The same, and each row r with keep_row[r] in [0, keep_rows) is also stored
+ * unencoded, in fp32, at k_keep / v_keep + keep_row[r] * head_dim (16-byte
+ * aligned buffers of keep_rows rows): the exact rows of a page that is still
+ * filling, which its final encode reads.  A row whose page id is outside the
+ * pool is only kept. */
+int dc_encode_rows_kv_keep(const void* k_values, const void* v_values, int32_t values_dtype, int64_t n_rows,
+                           int64_t row_stride, const int32_t* k_row_page, const int32_t* k_row_slot,
+                           const int32_t* v_row_page, const int32_t* v_row_slot, dc_pool k_pool, dc_pool v_pool,
+                           float* k_keep, float* v_keep, const int32_t* keep_row, int32_t keep_rows, dc_stream_t stream);
+
+/* Keys and values [n_streams][n_tokens] of token streams in one launch, the
+ * destinations from page tables: token t of stream s is token u = first_slot +
+ * t of the stream's table row and goes to slot u % page_tokens of page
+ * k_table / v_table[s * table_stride + u / page_tokens] (device int32; an id
+ * outside the pool: not encoded).  With k_keep / v_keep (NULL: none), tokens u
+ * >= keep_from are also stored in fp32 at row s * page_tokens + u %
+ * page_tokens (buffers of n_streams * page_tokens rows): a prompt's tail.  A
+ * prompt's ingest needs no per-row ids (reference
+ * dotcache/model_kv_cache.py:3609-3691). */
+int dc_encode_streams_kv(const void* k_values, const void* v_values, int32_t values_dtype, int32_t n_streams,
+                         int32_t n_tokens, int64_t row_stride, const int32_t* k_table, const int32_t* v_table,
+                         int32_t table_stride, int32_t first_slot, int32_t page_tokens, dc_pool k_pool, dc_pool v_pool,
+                         float* k_keep, float* v_keep, int32_t keep_from, dc_stream_t stream);
+
 /* Process-wide encode kernel choice: 0 (default) runs the wavefront kernel
  * (8 channels per lane, several rows per wavefront) wherever the pool's
  * geometry fits it, 1 always runs the general one-thread-per-group kernel
