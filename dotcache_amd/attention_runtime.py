@@ -36,6 +36,17 @@ def _resolve_backend(backend: BackendName, page: PageLike) -> Literal["hip_mi355
     return "hip_mi355x"
 
 
+def _resolve_pages(backend: BackendName, pages: Sequence[PageLike]) -> None:
+    """:func:`_resolve_backend` for every page.  A prepared page was checked
+    when it was prepared, so past the first page only host pages are."""
+    if not pages:
+        return
+    _resolve_backend(backend, pages[0])
+    for p in pages:
+        if not isinstance(p, PreparedPageHIP) and not hip.page_supported_hip(p):
+            raise ValueError("page is unsupported by hip_mi355x in this phase")
+
+
 def prepare_page(page: PageLike, *, backend: BackendName = "auto", cache: PreparedPageCache | None = None,
                  trace: ExecutionTrace | None = None) -> PreparedPageHIP:
     """Reference ``attention_runtime.py:72-87``: through ``cache`` when given."""
@@ -48,8 +59,7 @@ def prepare_page(page: PageLike, *, backend: BackendName = "auto", cache: Prepar
 def prepare_pages(pages: Sequence[PageLike], *, backend: BackendName = "auto",
                   cache: PreparedPageCache | None = None, trace: ExecutionTrace | None = None) -> list[PreparedPageHIP]:
     """Reference ``attention_runtime.py:90-108``."""
-    for p in pages:
-        _resolve_backend(backend, p)
+    _resolve_pages(backend, pages)
     if cache is not None:
         return cache.prepare_pages(list(pages), backend="hip_mi355x", trace=trace)
     return hip.prepare_pages_hip(pages, trace=trace)
@@ -70,8 +80,7 @@ def score_pages(query_slice, pages: Sequence[PageLike], *, backend: BackendName 
                 cache: PreparedPageCache | None = None, trace: ExecutionTrace | None = None) -> list[np.ndarray]:
     if not pages:
         return []
-    for p in pages:
-        _resolve_backend(backend, p)
+    _resolve_pages(backend, pages)
     return hip.score_pages_hip(query_slice, _cached(pages, backend, cache, trace), trace=trace)
 
 
@@ -110,8 +119,8 @@ def decode_multi_query_step(query_slices, key_pages: Sequence[PageLike], value_p
         raise ValueError("key_pages and value_pages must contain the same number of pages")
     if not key_pages:
         raise ValueError("decode_multi_query_step requires at least one page")
-    for p in list(key_pages) + list(value_pages):
-        _resolve_backend(backend, p)
+    _resolve_pages(backend, key_pages)
+    _resolve_pages(backend, value_pages)
     return hip.decode_multi_query_step_hip(queries, _cached(key_pages, backend, cache, trace),
                                            _cached(value_pages, backend, cache, trace), trace=trace)
 
@@ -126,8 +135,8 @@ def decode_step_with_page_logits(query_slice, key_pages: Sequence[PageLike], val
         raise ValueError("decode_step requires at least one page")
     if page_logits is not None and len(page_logits) != len(key_pages):
         raise ValueError("page_logits must align with key_pages")
-    for p in list(key_pages) + list(value_pages):
-        _resolve_backend(backend, p)
+    _resolve_pages(backend, key_pages)
+    _resolve_pages(backend, value_pages)
     return hip.decode_step_hip(query_slice, _cached(key_pages, backend, cache, trace),
                                _cached(value_pages, backend, cache, trace), precomputed_page_logits=page_logits,
                                trace=trace)

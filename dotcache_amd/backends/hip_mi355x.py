@@ -37,7 +37,7 @@ from typing import Any, Sequence
 import numpy as np
 
 from .. import _lib
-from ..decode import decode_paged
+from ..decode import chunks_per_page, decode_paged, launch_lead_ratio, launch_target_items, make_plan
 from ..page_pool import DevicePagePool, PoolGeometry, current_stream_ptr, page_format_of
 from ..tracing import ExecutionTrace
 from ..types import EncodedPage, PageHeader
@@ -202,8 +202,9 @@ def _one_pool(pages: Sequence[PageLike], trace=None) -> tuple[DevicePagePool, np
     """Prepared pages that all live in one pool (re-preparing into the
     largest-capacity pool when they do not)."""
     prepared = prepare_pages_hip(pages, trace=trace)
-    pools = {id(p.pool): p.pool for p in prepared}
-    if len(pools) > 1:
+    pool = prepared[0].pool
+    if any(p.pool is not pool for p in prepared):
+        pools = {id(p.pool): p.pool for p in prepared}
         target = max(pools.values(), key=lambda pl: pl.geometry.page_capacity)
         prepared = prepare_pages_hip([p.source_page if p.pool is not target else p for p in prepared], trace=trace,
                                      pool=target)
@@ -228,6 +229,31 @@ def _record_reads(trace: ExecutionTrace | None, prepared: Sequence[PreparedPageH
         trace.record_device_read(p.source_page.device_nbytes)
 
 
+class _Upload:
+    """Small host arrays on the device in one copy: ``_Upload(dev, a, b).ptr``
+    holds their device addresses, 16-byte aligned, valid while it lives (and,
+    for work queued on this stream, after)."""
+
+    def __init__(self, device, *arrays: np.ndarray):
+        at, end = [], 0
+        for x in arrays:
+            at.append(end)
+            end += -(-x.nbytes // 16) * 16
+        buf = np.empty(max(end, 16), dtype=np.uint8)
+        for o, x in zip(at, arrays):
+            buf[o: o + x.nbytes] = np.ascontiguousarray(x).reshape(-1).view(np.uint8)
+        self.data = _torch().from_numpy(buf).to(device)
+        base = self.data.data_ptr()
+        self.ptr = [base + o for o in at]
+
+
+def _starts(tokens: np.ndarray) -> np.ndarray:
+    """int32 ``[n + 1]`` running token counts."""
+    out = np.zeros(tokens.size + 1, dtype=np.int32)
+    np.cumsum(tokens, out=out[1:])
+    return out
+
+
 def _queries_tensor(q, hd: int, device):
     torch = _torch()
     t = q if isinstance(q, torch.Tensor) else torch.as_tensor(np.asarray(q, dtype=np.float32))
@@ -239,25 +265,35 @@ def _queries_tensor(q, hd: int, device):
     return t.contiguous()
 
 
-def _score_tensor(queries, pool: DevicePagePool, ids: np.ndarray, score=None):
-    """logits [n_queries, total_tokens] on the device.  With ``score`` (a
-    bool mask over the pages), only those pages are scored; the columns of
-    the others are left unwritten."""
+def _host_queries(q, hd: int):
+    """fp32 numpy ``[n, hd]`` for queries on the host, None for device tensors."""
+    torch = _torch()
+    if isinstance(q, torch.Tensor):
+        if q.device.type != "cpu":
+            return None
+        q = q.detach().to(torch.float32).numpy()
+    a = np.asarray(q, dtype=np.float32)
+    if a.ndim == 1:
+        a = a[None, :]
+    if a.shape[-1] != hd:
+        raise ValueError("query head_dim does not match the pages")
+    return a
+
+
+def _score_tensor(queries, pool: DevicePagePool, ids: np.ndarray):
+    """logits [n_queries, total_tokens] on the device."""
     torch = _torch()
     dev = pool.device
-    tok = pool.tokens_of(ids)
-    offsets = np.zeros(ids.size + 1, dtype=np.int32)
-    offsets[1:] = np.cumsum(tok)
+    offsets = _starts(pool.tokens_of(ids))
     total = int(offsets[-1])
-    q = _queries_tensor(queries, pool.geometry.head_dim, dev)
+    qh = _host_queries(queries, pool.geometry.head_dim)
+    q = _queries_tensor(queries, pool.geometry.head_dim, dev) if qh is None else qh
     logits = torch.empty((q.shape[0], total), dtype=torch.float32, device=dev)
-    sel_ids, sel_off = (ids, offsets) if score is None else (ids[score], offsets[:-1][score])
-    if sel_ids.size:
-        ids_d = torch.from_numpy(np.ascontiguousarray(sel_ids)).to(dev)
-        off_d = torch.from_numpy(np.ascontiguousarray(sel_off)).to(dev)
-        st = _lib.lib().dc_score_pages(pool.c_pool(), C.c_void_p(ids_d.data_ptr()), C.c_void_p(off_d.data_ptr()),
-                                       sel_ids.size, C.c_void_p(q.data_ptr()), q.shape[0],
-                                       C.c_void_p(logits.data_ptr()), total, C.c_void_p(current_stream_ptr()))
+    if ids.size:
+        up = _Upload(dev, ids, offsets, *([] if qh is None else [qh]))
+        st = _lib.lib().dc_score_pages(pool.c_pool(), up.ptr[0], up.ptr[1], ids.size,
+                                       q.data_ptr() if qh is None else up.ptr[2], q.shape[0], logits.data_ptr(), total,
+                                       current_stream_ptr())
         _lib.check(st, "dc_score_pages")
     return logits, offsets
 
@@ -266,9 +302,7 @@ def _mix_tensor(weights, pool: DevicePagePool, ids: np.ndarray, out=None):
     """out [n_queries, head_dim] (+)= weights [n_queries, total_tokens] @ V."""
     torch = _torch()
     dev = pool.device
-    tok = pool.tokens_of(ids)
-    offsets = np.zeros(ids.size + 1, dtype=np.int32)
-    offsets[1:] = np.cumsum(tok)
+    offsets = _starts(pool.tokens_of(ids))
     w = weights if isinstance(weights, torch.Tensor) else torch.as_tensor(np.asarray(weights, dtype=np.float32))
     w = w.to(device=dev, dtype=torch.float32)
     if w.dim() == 1:
@@ -280,23 +314,11 @@ def _mix_tensor(weights, pool: DevicePagePool, ids: np.ndarray, out=None):
     if out is None:
         out = torch.empty((w.shape[0], pool.geometry.head_dim), dtype=torch.float32, device=dev)
         acc = 0
-    ids_d = torch.from_numpy(ids).to(dev)
-    off_d = torch.from_numpy(offsets).to(dev)
-    st = _lib.lib().dc_mix_pages(pool.c_pool(), C.c_void_p(ids_d.data_ptr()), C.c_void_p(off_d.data_ptr()), ids.size,
-                                 C.c_void_p(w.data_ptr()), w.shape[0], w.shape[1], C.c_void_p(out.data_ptr()), acc,
-                                 C.c_void_p(current_stream_ptr()))
+    up = _Upload(dev, ids, offsets)
+    st = _lib.lib().dc_mix_pages(pool.c_pool(), up.ptr[0], up.ptr[1], ids.size, w.data_ptr(), w.shape[0], w.shape[1],
+                                 out.data_ptr(), acc, current_stream_ptr())
     _lib.check(st, "dc_mix_pages")
     return out
-
-
-def _softmax(x):
-    """Softmax of the rows of fp32 ``x [..., n]`` (contiguous) in a new tensor."""
-    y = _torch().empty_like(x)
-    n = x.shape[-1]
-    st = _lib.lib().dc_softmax_rows_to(C.c_void_p(x.data_ptr()), n, C.c_void_p(y.data_ptr()), n,
-                                       x.numel() // n if n else 0, n, C.c_void_p(current_stream_ptr()))
-    _lib.check(st, "dc_softmax_rows_to")
-    return y
 
 
 def score_page_hip(query_slice: np.ndarray | Any, page: PageLike, *, trace: ExecutionTrace | None = None) -> np.ndarray:
@@ -347,15 +369,10 @@ def _pair_pools(key_pages, value_pages, trace):
     return kpool, vpool, kid, vid, kprep + vprep
 
 
-def decode_multi_query_step_hip_tensor(query_slices, key_pages, value_pages, *, precomputed_page_logits=None,
-                                       trace: ExecutionTrace | None = None):
-    """(logits [Q, T], weights [Q, T], output [Q, head_dim]) as device tensors.
-
-    ``precomputed_page_logits[i]``, when not None, is used as page i's logits
-    and page i's key bytes are not read (reference
-    ``decode_step_with_page_logits``, dotcache/attention_runtime.py:298-303,
-    and its device path dotcache/backends/torch_mps.py:2690-2700); the trace
-    counts the key pages scored and every value page."""
+def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits, trace):
+    """(flat, Q, T, head_dim): logits [Q, T], weights [Q, T] and output [Q,
+    head_dim] one after the other in a flat fp32 device tensor (so that one
+    copy takes all three to the host)."""
     torch = _torch()
     kpool, vpool, kid, vid, prepared = _pair_pools(key_pages, value_pages, trace)
     kprep, vprep = prepared[:kid.size], prepared[kid.size:]
@@ -365,38 +382,94 @@ def decode_multi_query_step_hip_tensor(query_slices, key_pages, value_pages, *, 
             raise ValueError("precomputed_page_logits must align with key_pages")
         cached = list(precomputed_page_logits)
     score = np.asarray([c is None for c in cached], dtype=bool)
-    kread = [p for p, s in zip(kprep, score) if s]
-    _record_reads(trace, kread + list(vprep), "decode_multi_query_step")
-    logits, offsets = _score_tensor(query_slices, kpool, kid, score=None if score.all() else score)
-    for i, c in enumerate(cached):
-        if c is None:
-            continue
-        c = torch.as_tensor(np.asarray(c, dtype=np.float32) if not isinstance(c, torch.Tensor) else c,
-                            dtype=torch.float32, device=kpool.device)
-        n = int(offsets[i + 1] - offsets[i])
-        if c.numel() != n:
-            raise ValueError("precomputed page logits must have shape [token_count]")
-        logits[:, offsets[i]: offsets[i + 1]] = c.reshape(1, n)
-    weights = _softmax(logits)
-    out = _mix_tensor(weights, vpool, vid)
-    return logits, weights, out
+    every = bool(score.all())
+    _record_reads(trace, list(kprep if every else [p for p, s in zip(kprep, score) if s]) + list(vprep),
+                  "decode_multi_query_step")
+    dev, hd = kpool.device, kpool.geometry.head_dim
+    offsets = _starts(kpool.tokens_of(kid))
+    T = int(offsets[-1])
+    qh = _host_queries(query_slices, hd)
+    q = _queries_tensor(query_slices, hd, dev) if qh is None else qh
+    Q = int(q.shape[0])
+    flat = torch.empty(2 * Q * T + Q * vpool.geometry.head_dim, dtype=torch.float32, device=dev)
+    logits = flat[: Q * T].view(Q, T)
+    sid, soff = (kid, offsets) if every else (kid[score], offsets[:-1][score])
+    up = _Upload(dev, sid, soff, vid, offsets, *([] if qh is None else [qh]))
+    q_ptr = q.data_ptr() if qh is None else up.ptr[4]
+    L, stream, base = _lib.lib(), current_stream_ptr(), flat.data_ptr()
+    if sid.size:
+        _lib.check(L.dc_score_pages(kpool.c_pool(), up.ptr[0], up.ptr[1], sid.size, q_ptr, Q, base, T, stream),
+                   "dc_score_pages")
+    if not every:
+        columns, values = [], []
+        for i in np.flatnonzero(~score).tolist():
+            c = cached[i]
+            n = int(offsets[i + 1] - offsets[i])
+            if isinstance(c, torch.Tensor) and c.device.type != "cpu":
+                c = c.to(device=dev, dtype=torch.float32)
+                if c.numel() != n:
+                    raise ValueError("precomputed page logits must have shape [token_count]")
+                logits[:, offsets[i]: offsets[i + 1]] = c.reshape(1, n)
+                continue
+            c = np.asarray(c, dtype=np.float32).reshape(-1)
+            if c.size != n:
+                raise ValueError("precomputed page logits must have shape [token_count]")
+            columns.append(np.arange(offsets[i], offsets[i + 1], dtype=np.int64))
+            values.append(c)
+        if columns:
+            logits[:, torch.from_numpy(np.concatenate(columns)).to(dev)] = torch.from_numpy(np.concatenate(values)).to(dev)
+    if T:
+        _lib.check(L.dc_softmax_rows_to(base, T, base + 4 * Q * T, T, Q, T, stream), "dc_softmax_rows_to")
+    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, base + 4 * Q * T, Q, T, base + 8 * Q * T, 0,
+                              stream), "dc_mix_pages")
+    return flat, Q, T, int(vpool.geometry.head_dim)
+
+
+def _split(flat, Q: int, T: int, hd: int):
+    return flat[: Q * T].reshape(Q, T), flat[Q * T: 2 * Q * T].reshape(Q, T), flat[2 * Q * T:].reshape(Q, hd)
+
+
+def decode_multi_query_step_hip_tensor(query_slices, key_pages, value_pages, *, precomputed_page_logits=None,
+                                       trace: ExecutionTrace | None = None):
+    """(logits [Q, T], weights [Q, T], output [Q, head_dim]) as device tensors.
+
+    ``precomputed_page_logits[i]``, when not None, is used as page i's logits
+    and page i's key bytes are not read (reference
+    ``decode_step_with_page_logits``, dotcache/attention_runtime.py:298-303,
+    and its device path dotcache/backends/torch_mps.py:2690-2700); the trace
+    counts the key pages scored and every value page."""
+    return _split(*_decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits, trace))
 
 
 def decode_step_hip(query_slice, key_pages, value_pages, *, precomputed_page_logits=None,
                     trace: ExecutionTrace | None = None) -> tuple[np.ndarray, np.ndarray, np.ndarray]:
     """(logits, weights, output) for one query -- reference ``decode_step_cuda``."""
     q = np.asarray(query_slice, dtype=np.float32) if not hasattr(query_slice, "device") else query_slice
-    logits, weights, out = decode_multi_query_step_hip_tensor(q, key_pages, value_pages,
-                                                              precomputed_page_logits=precomputed_page_logits, trace=trace)
-    return logits[0].cpu().numpy(), weights[0].cpu().numpy(), out[0].cpu().numpy()
+    flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, precomputed_page_logits, trace)
+    logits, weights, out = _split(flat.cpu().numpy(), Q, T, hd)
+    return logits[0].copy(), weights[0].copy(), out[0].copy()
 
 
 def decode_multi_query_step_hip(query_slices, key_pages, value_pages, *, trace: ExecutionTrace | None = None):
     q = np.asarray(query_slices, dtype=np.float32) if not hasattr(query_slices, "device") else query_slices
     if getattr(q, "ndim", 2) != 2:
         raise ValueError("query_slices must have shape [query_count, head_dim]")
-    logits, weights, out = decode_multi_query_step_hip_tensor(q, key_pages, value_pages, trace=trace)
-    return logits.cpu().numpy(), weights.cpu().numpy(), out.cpu().numpy()
+    flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, None, trace)
+    logits, weights, out = _split(flat.cpu().numpy(), Q, T, hd)
+    return logits.copy(), weights.copy(), out.copy()
+
+
+def _group_queries(query_groups, hd: int, device):
+    """(queries [G, Q, hd], host array or None): one fp32 numpy array when every
+    group's queries are on the host, else a device tensor."""
+    torch = _torch()
+    host = [_host_queries(x, hd) for x in query_groups]
+    if all(x is not None for x in host):
+        if len({x.shape for x in host}) != 1:
+            raise RuntimeError("every query group must hold the same number of queries")
+        q = np.stack(host)
+        return q, q
+    return torch.stack([_queries_tensor(x, hd, device) for x in query_groups]), None
 
 
 def _grouped_inputs(query_groups, key_pages_by_group, value_pages_by_group):
@@ -434,34 +507,29 @@ def decode_grouped_multiquery_step_prepared_hip_tensor(query_groups, key_pages_b
         raise ValueError("key and value pages must hold the same token counts")
     bounds = np.zeros(G + 1, dtype=np.int64)
     bounds[1:] = np.cumsum(counts)
-    totals = [int(ktok[bounds[g]:bounds[g + 1]].sum()) for g in range(G)]
+    totals = np.diff(_starts(ktok)[bounds]).tolist()
     dev = kpool.device
-    q = torch.stack([_queries_tensor(x, kpool.geometry.head_dim, dev) for x in query_groups]).contiguous()  # [G, Q, hd]
+    q, qh = _group_queries(query_groups, kpool.geometry.head_dim, dev)
     Q, hd = int(q.shape[1]), int(q.shape[2])
     if len(set(totals)) != 1:
         raise ValueError("all query groups must have the same query count and token count for batched grouped decode")
     T = totals[0]
     # first token of every page within its group, the group of every page
-    starts = np.zeros(len(kids), dtype=np.int32)
-    for g in range(G):
-        seg = ktok[bounds[g]:bounds[g + 1]]
-        starts[bounds[g]:bounds[g + 1]] = np.cumsum(seg) - seg
+    ends = np.cumsum(ktok)
+    starts = (ends - ktok - np.repeat(np.arange(G) * T, counts)).astype(np.int32)
     page_group = np.repeat(np.arange(G, dtype=np.int32), counts)
-    kids_d, vids_d = torch.from_numpy(kids).to(dev), torch.from_numpy(vids).to(dev)
-    off_d = torch.from_numpy(starts).to(dev)
-    grp_d = torch.from_numpy(page_group).to(dev)
-    gp_d = torch.from_numpy(bounds.astype(np.int32)).to(dev)
+    up = _Upload(dev, kids, vids, starts, page_group, bounds.astype(np.int32), *([] if qh is None else [qh]))
     logits = torch.empty((G, Q, T), dtype=torch.float32, device=dev)
-    stream = C.c_void_p(current_stream_ptr())
-    L = _lib.lib()
-    _lib.check(L.dc_score_pages_grouped(kpool.c_pool(), C.c_void_p(kids_d.data_ptr()), C.c_void_p(off_d.data_ptr()),
-                                        C.c_void_p(grp_d.data_ptr()), G, len(kids), C.c_void_p(q.data_ptr()), Q,
-                                        C.c_void_p(logits.data_ptr()), T, stream), "dc_score_pages_grouped")
-    weights = _softmax(logits)
+    weights = torch.empty((G, Q, T), dtype=torch.float32, device=dev)
     out = torch.empty((G, Q, hd), dtype=torch.float32, device=dev)
-    _lib.check(L.dc_mix_pages_grouped(vpool.c_pool(), C.c_void_p(vids_d.data_ptr()), C.c_void_p(off_d.data_ptr()),
-                                      C.c_void_p(gp_d.data_ptr()), G, len(vids), C.c_void_p(weights.data_ptr()), Q, T,
-                                      C.c_void_p(out.data_ptr()), 0, stream), "dc_mix_pages_grouped")
+    L, stream = _lib.lib(), current_stream_ptr()
+    _lib.check(L.dc_score_pages_grouped(kpool.c_pool(), up.ptr[0], up.ptr[2], up.ptr[3], G, len(kids),
+                                        q.data_ptr() if qh is None else up.ptr[5], Q, logits.data_ptr(), T, stream),
+               "dc_score_pages_grouped")
+    if T:
+        _lib.check(L.dc_softmax_rows_to(logits.data_ptr(), T, weights.data_ptr(), T, G * Q, T, stream), "dc_softmax_rows_to")
+    _lib.check(L.dc_mix_pages_grouped(vpool.c_pool(), up.ptr[1], up.ptr[2], up.ptr[4], G, len(vids), weights.data_ptr(), Q,
+                                      T, out.data_ptr(), 0, stream), "dc_mix_pages_grouped")
     return logits, weights, out
 
 
@@ -489,6 +557,8 @@ def decode_grouped_multiquery_step_prepared_hip_tensor_output_only(query_groups,
     if vpool.geometry.page_capacity != kpool.geometry.page_capacity:
         vpool, vids, vprep = _one_pool_with_capacity(flat_v, kpool.geometry.page_capacity, trace)
     _record_reads(trace, kprep + vprep, "decode_grouped_output_only")
+    if not np.array_equal(kpool.tokens_of(kids), vpool.tokens_of(vids)):
+        raise ValueError("key and value pages must hold the same token counts")
     width = max(counts)
     kt = np.zeros((G, 1, width), dtype=np.int32)  # one "sequence" per group with one KV head
     vt = np.zeros((G, 1, width), dtype=np.int32)
@@ -498,8 +568,21 @@ def decode_grouped_multiquery_step_prepared_hip_tensor_output_only(query_groups,
         vt[g, 0, :n] = vids[off: off + n]
         off += n
     dev = kpool.device
-    q = torch.stack([_queries_tensor(x, kpool.geometry.head_dim, dev) for x in query_groups])  # [G, Q, hd]
-    out = decode_paged(kpool, torch.from_numpy(kt).to(dev), torch.from_numpy(vt).to(dev),
-                       np.asarray(counts, dtype=np.int32), q[:, None].contiguous(), pages_per_split=pages_per_split,
-                       v_pool=vpool)
+    q, qh = _group_queries(query_groups, kpool.geometry.head_dim, dev)
+    if qh is not None:
+        q = torch.from_numpy(qh).to(dev)
+    tables = torch.from_numpy(np.stack([kt, vt])).to(dev)
+    seq_pages = np.asarray(counts, dtype=np.int32)
+    # (what decode_paged would check by reading the tables back)
+    kpool.validate_ids(kids)
+    vpool.validate_ids(vids)
+    plan = None
+    if pages_per_split is None:
+        last = kpool.tokens_of(kt[np.arange(G), 0, seq_pages - 1]).astype(np.int32)
+        Q = int(q.shape[1])
+        plan = make_plan(seq_pages, 1, device=dev, chunks_per_page=chunks_per_page(kpool.geometry.page_capacity),
+                         target_items=launch_target_items(kpool, vpool, Q), last_page_tokens=last,
+                         lead_ratio=launch_lead_ratio(kpool, vpool, Q))
+    out = decode_paged(kpool, tables[0], tables[1], seq_pages, q[:, None].contiguous(), pages_per_split=pages_per_split,
+                       plan=plan, v_pool=vpool, validate=False)
     return out[:, 0]

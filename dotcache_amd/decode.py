@@ -15,6 +15,7 @@ steady decode loop uploads nothing.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 from dataclasses import dataclass
 
 import numpy as np
@@ -140,10 +141,15 @@ def default_target_items() -> int:
     try:
         torch = _torch()
         if torch.cuda.is_available():
-            return 4 * int(torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count)
+            return _simds(torch.cuda.current_device())
     except Exception:
         pass
     return DEFAULT_TARGET_ITEMS
+
+
+@functools.lru_cache(maxsize=None)
+def _simds(device: int) -> int:
+    return 4 * int(_torch().cuda.get_device_properties(device).multi_processor_count)
 
 
 def waves_per_simd(pool: DevicePagePool, v_pool: DevicePagePool | None, n_q: int, k_mask: int | None = None,
@@ -153,11 +159,10 @@ def waves_per_simd(pool: DevicePagePool, v_pool: DevicePagePool | None, n_q: int
     ``v_mask``: the formats of the pages the launch reads
     (``format_mask_of``), when narrower than the pools'."""
     vpool = pool if v_pool is None else v_pool
-    kp, vp = pool.c_pool(), vpool.c_pool()
-    if k_mask:
-        kp.format_mask = int(k_mask) & pool.format_mask
-    if v_mask:
-        vp.format_mask = int(v_mask) & vpool.format_mask
+    # (the choice reads the geometries and format masks only)
+    kp, vp = _lib.Pool(geometry=pool.geometry.c()), _lib.Pool(geometry=vpool.geometry.c())
+    kp.format_mask = int(k_mask) & pool.format_mask if k_mask else pool.format_mask
+    vp.format_mask = int(v_mask) & vpool.format_mask if v_mask else vpool.format_mask
     return int(_lib.lib().dc_decode_waves_per_simd(kp, vp, int(n_q)))
 
 
@@ -598,9 +603,9 @@ def make_region_plan(seq_pages, n_kv_heads: int, front, *, device="cuda", chunks
         raise ValueError("page_cost must have shape [n_seqs, n_kv_heads, >= max pages]")
     target = int(target_items) if target_items else default_target_items()
     if window_merge:
-        wtok = [sum(full if p + 1 < sp[b] else int(last[b]) for p in range(int(fr[b, 0]), int(fr[b, 1])))
-                for b in range(B)]
-        if np.any(fr[:, 1] - fr[:, 0] > 8) or max(wtok) > 256:
+        width = fr[:, 1] - fr[:, 0]
+        wtok = width * full - np.where((width > 0) & (fr[:, 1] == sp), full - last, 0)
+        if np.any(width > 8) or int(wtok.max()) > 256:
             raise ValueError("window_merge: a window holds at most 256 tokens in at most 8 pages")
         if np.any((fr[:, 0] == 0) & (fr[:, 1] == sp)):
             raise ValueError("window_merge: every stream needs pages outside its window")
@@ -783,18 +788,19 @@ def merge_windows(pool: DevicePagePool, vpool: DevicePagePool, kt: np.ndarray, v
     if pool.geometry.head_dim not in (64, 128, 256):
         return None
     f16 = _lib.FMT_M3_F16
-    out = np.zeros((kt.shape[0], 2), dtype=np.int64)
-    for b in range(kt.shape[0]):
-        n = int(seq_pages[b])
-        exact = (pool.formats_of(kt[b, :, :n]) == f16) & (vpool.formats_of(vt[b, :, :n]) == f16)
-        if not np.all(exact == exact[0]):
-            return None
-        run = n - int(np.flatnonzero(~exact[0])[-1]) - 1 if not exact[0].all() else n
-        begin = n - run
-        if run and (begin == 0 or run > 8 or int(pool.tokens_of(kt[b, :, begin:n]).sum(axis=-1).max()) > 256):
-            return None
-        out[b] = (begin, n)
-    return out if np.any(out[:, 1] > out[:, 0]) else None
+    n = np.asarray(seq_pages, dtype=np.int64)
+    page = np.arange(kt.shape[2])
+    live = page < n[:, None]
+    exact = (pool.formats_of(kt) == f16) & (vpool.formats_of(vt) == f16) & live[:, None, :]
+    if not np.all(exact == exact[:, :1]):
+        return None
+    # the run starts after the last page that is not exact
+    begin = np.where(live & ~exact[:, 0], page + 1, 0).max(axis=1, initial=0)
+    run = n - begin
+    tokens = np.where((page >= begin[:, None, None]) & live[:, None, :], pool.tokens_of(kt), 0).sum(axis=2).max(axis=1)
+    if np.any((run > 0) & ((begin == 0) | (run > 8) | (tokens > 256))) or not np.any(run > 0):
+        return None
+    return np.stack([begin, n], axis=1)
 
 
 def plan_decode(pool: DevicePagePool, vpool: DevicePagePool, kt: np.ndarray, vt: np.ndarray, seq_pages, n_q: int, *,
@@ -815,8 +821,9 @@ def plan_decode(pool: DevicePagePool, vpool: DevicePagePool, kt: np.ndarray, vt:
         read = read & ~((pg >= front[:, 0, None, None]) & (pg < front[:, 1, None, None]))
     read = np.broadcast_to(read, kt.shape)
     masks = (pool.format_mask_of(kt[read]) & pool.format_mask, vpool.format_mask_of(vt[read]) & vpool.format_mask)
-    target = launch_target_items(pool, vpool, n_q, *masks)
-    lead = launch_lead_ratio(pool, vpool, n_q, *masks)
+    waves = waves_per_simd(pool, vpool, n_q, *masks)
+    target = default_target_items() * waves
+    lead = LEAD_RATIO if waves == 2 else None
     if front is not None:
         plan = make_region_plan(sp, H, front, device=device, chunks_per_page=cpp, target_items=target,
                                 last_page_tokens=last_page_tokens, window_merge=True, lead_ratio=lead)
@@ -945,7 +952,7 @@ def decode_paged(
     if records is not None and not records.fresh_for(plan, k_table, v_table, pool, vpool):
         raise ValueError("page records are stale: gather them again after a change to the plan, the page "
                          "tables or the pools' descriptors")
-    stream = C.c_void_p(current_stream_ptr())
+    stream = current_stream_ptr()
 
     def launch(first: int, count: int, with_merges: bool, masks) -> None:
         """Items [first, first + count) in one launch (and the plan's merges
@@ -960,16 +967,14 @@ def decode_paged(
             # (records checked fresh above: the masks are those of these tables' pages)
             kp.format_mask, vp.format_mask = masks
         m_on = with_merges and merge and plan.merges is not None
-        args = (kp, vp, C.c_void_p(k_table.data_ptr()), C.c_void_p(v_table.data_ptr()), stride,
-                C.c_void_p(plan.items.data_ptr() + 32 * first), count,
-                C.c_void_p(plan.merges.data_ptr() if m_on else 0), plan.n_merges if m_on else 0,
-                C.c_void_p(queries.data_ptr()), dtype_code(queries), float(query_scale),
-                B, H, Q, C.c_void_p(out.data_ptr()), C.c_void_p(workspace.data_ptr()), int(workspace.numel()))
+        args = (kp, vp, k_table.data_ptr(), v_table.data_ptr(), stride, plan.items.data_ptr() + 32 * first, count,
+                plan.merges.data_ptr() if m_on else None, plan.n_merges if m_on else 0, queries.data_ptr(),
+                dtype_code(queries), float(query_scale), B, H, Q, out.data_ptr(), workspace.data_ptr(), workspace.numel())
         if records is None:
             st = _lib.lib().dc_decode_paged(*args, stream)
         else:
-            st = _lib.lib().dc_decode_paged_records(
-                *args, C.c_void_p(records.data.data_ptr() + 16 * records.stride * first), records.stride, stream)
+            st = _lib.lib().dc_decode_paged_records(*args, records.data.data_ptr() + 16 * records.stride * first,
+                                                    records.stride, stream)
         _lib.check(st, "dc_decode_paged")
 
     nf = int(plan.n_front)

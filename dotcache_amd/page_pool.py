@@ -21,6 +21,7 @@ in ``libdotcache_hip.so``.
 from __future__ import annotations
 
 import ctypes as C
+import functools
 from collections import deque
 from dataclasses import dataclass, replace
 
@@ -72,14 +73,13 @@ def page_format_of(mode: str, scheme: str, bits: int, escape_dtype: str = "float
 
 
 def dtype_code(t) -> int:
-    torch = _torch()
-    if t.dtype == torch.float32:
-        return _lib.DT_F32
-    if t.dtype == torch.float16:
-        return _lib.DT_F16
-    if t.dtype == torch.bfloat16:
-        return _lib.DT_BF16
-    raise ValueError(f"unsupported tensor dtype {t.dtype}")
+    if not _TORCH_DT:
+        torch = _torch()
+        _TORCH_DT.update({torch.float32: _lib.DT_F32, torch.float16: _lib.DT_F16, torch.bfloat16: _lib.DT_BF16})
+    code = _TORCH_DT.get(t.dtype)
+    if code is None:
+        raise ValueError(f"unsupported tensor dtype {t.dtype}")
+    return code
 
 
 def current_stream_ptr() -> int:
@@ -97,8 +97,12 @@ class PoolGeometry:
     def num_groups(self) -> int:
         return -(-self.head_dim // self.group_size)
 
-    def c(self) -> _lib.PageGeometry:
+    @functools.cached_property
+    def _c(self) -> _lib.PageGeometry:
         return _lib.geometry(self.head_dim, self.group_size, self.page_capacity, self.layout)
+
+    def c(self) -> _lib.PageGeometry:
+        return self._c
 
 
 class _PageHeaders(dict):
@@ -371,10 +375,8 @@ class DevicePagePool:
 
     def c_pool(self) -> _lib.Pool:
         descs = self.device_descs()
-        return _lib.Pool(
-            C.c_void_p(self.arena.data_ptr()), self.arena.numel(), C.c_void_p(descs.data_ptr()), self._n_pages,
-            self.geometry.c(), self.format_mask,
-        )
+        return _lib.Pool(self.arena.data_ptr(), self.arena.numel(), descs.data_ptr(), self._n_pages, self.geometry.c(),
+                         self.format_mask)
 
     # ---- host <-> device pages --------------------------------------------
     def _check_page_geometry(self, page: EncodedPage) -> None:

@@ -40,17 +40,18 @@ def select_window_page_indices(key_pages: Sequence[PageLike], *, recent_window_t
     page end (reference ``session_runtime.py:189-216``)."""
     if not key_pages:
         return []
-    end = max(p.header.token_start + p.header.token_count for p in key_pages)
+    headers = [p.header for p in key_pages]
+    start = np.asarray([h.token_start for h in headers], dtype=np.int64)
+    stop = start + np.asarray([h.token_count for h in headers], dtype=np.int64)
+    end = int(stop.max())
     sink = max(0, int(sink_window_tokens))
     recent = int(recent_window_tokens) if recent_window_tokens is not None else 0
-    recent_start = max(0, end - recent) if recent > 0 else end
-    out = []
-    for i, p in enumerate(key_pages):
-        start = p.header.token_start
-        stop = start + p.header.token_count
-        if (sink > 0 and start < sink and stop > 0) or (recent > 0 and stop > recent_start):
-            out.append(i)
-    return out
+    chosen = np.zeros(len(headers), dtype=bool)
+    if sink > 0:
+        chosen |= (start < sink) & (stop > 0)
+    if recent > 0:
+        chosen |= stop > max(0, end - recent)
+    return np.flatnonzero(chosen).tolist()
 
 
 def _stack_rows(arrays, n_rows: int | None = None) -> np.ndarray:

@@ -1,0 +1,90 @@
+"""Host-side rules that batched calls share with page-by-page ones: merge
+windows and page bookkeeping, over the forms they accept (no GPU)."""
+import numpy as np
+import pytest
+
+from dotcache_amd import _lib
+from dotcache_amd.decode import merge_windows
+from dotcache_amd.page_pool import DevicePagePool, PoolGeometry
+
+
+def _pool(cap=64, hd=64):
+    return DevicePagePool(PoolGeometry(hd, 32, cap), device="cpu", reserve_bytes=1 << 16, reserve_pages=16)
+
+
+def _windows_by_sequence(pool, vpool, kt, vt, seq_pages):
+    """The rule stated one sequence at a time."""
+    f16 = _lib.FMT_M3_F16
+    out = []
+    for b, n in enumerate(seq_pages):
+        exact = [[pool.formats_of(kt[b, h, p]) == f16 and vpool.formats_of(vt[b, h, p]) == f16 for p in range(n)]
+                 for h in range(kt.shape[1])]
+        if any(e != exact[0] for e in exact):
+            return None
+        begin = n
+        while begin > 0 and exact[0][begin - 1]:
+            begin -= 1
+        tokens = max(sum(int(pool.tokens_of(kt[b, h, p])) for p in range(begin, n)) for h in range(kt.shape[1]))
+        if begin < n and (begin == 0 or n - begin > 8 or tokens > 256):
+            return None
+        out.append((begin, n))
+    return np.asarray(out) if any(b < n for b, n in out) else None
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_merge_windows_match_the_rule_per_sequence(seed):
+    rng = np.random.default_rng(seed)
+    B, H, S = int(rng.integers(1, 5)), int(rng.integers(1, 4)), int(rng.integers(1, 14))
+    k, v = _pool(), _pool()
+    seq = rng.integers(1, S + 1, size=B)
+    kt, vt = (np.zeros((B, H, S), dtype=np.int32) for _ in range(2))
+    for b in range(B):
+        run = int(rng.integers(0, min(10, seq[b]) + 1)) * int(rng.random() < 0.8)
+        for p in range(S):
+            exact = seq[b] - run <= p < seq[b]
+            tokens = int(rng.integers(1, 65)) if rng.random() < 0.5 else 64
+            for h in range(H):
+                fmt = (_lib.FMT_M3_F16, 0) if exact != (rng.random() < 0.01) else (_lib.FMT_M0_AFFINE, 4)
+                kt[b, h, p] = k.allocate(*fmt, tokens=tokens)[0]
+                vt[b, h, p] = v.allocate(*fmt, tokens=tokens)[0]
+    got, want = merge_windows(k, v, kt, vt, seq), _windows_by_sequence(k, v, kt, vt, seq)
+    assert (got is None) == (want is None)
+    if want is not None:
+        np.testing.assert_array_equal(got, want)
+
+
+def test_pool_reuses_blobs_and_ids_in_order():
+    pool = _pool()
+    a = pool.allocate(_lib.FMT_M0_AFFINE, 4, 3, tokens=64)
+    b = pool.allocate(_lib.FMT_M3_F16, 0, 2, tokens=1)
+    starts = pool.descs_of(a)["block"].tolist()
+    pool.free([a[0], b[0], a[2]])
+    with pytest.raises(RuntimeError, match="not live"):
+        pool.free([a[1], a[0]])
+    assert pool.formats_of([a[1]])[0] == _lib.FMT_M0_AFFINE  # nothing was freed
+    with pytest.raises(RuntimeError):
+        pool.free([a[1], a[1]])
+    c = pool.allocate(_lib.FMT_M0_AFFINE, 4, 3, tokens=2)
+    assert c.tolist() == [a[0], b[0], a[2]]                       # ids oldest freed first
+    assert pool.descs_of(c)["block"].tolist()[:2] == [starts[2], starts[0]]  # blobs last freed first
+    assert pool.format_mask_of(c) == _lib.format_bit(_lib.FMT_M0_AFFINE, 4)
+    many = pool.allocate(_lib.FMT_M0_SYMMETRIC, 8, 40, tokens=3)  # past the reserved descriptors
+    assert len(set(many.tolist())) == 40 and (pool.tokens_of(many) == 3).all()
+
+
+def test_deferred_headers_are_made_once_and_follow_token_counts():
+    from dotcache_amd.config import DotCacheConfig
+    from dotcache_amd.encode import make_header, resolve_encode_spec
+
+    pool, cfg = _pool(), DotCacheConfig(head_dim=64)
+    ids = pool.allocate(_lib.FMT_M0_AFFINE, 4, 3, tokens=64).tolist()
+    template = make_header(cfg, resolve_encode_spec(cfg, kind="K"), kind="K", layer_id=0, kv_head_id=0, token_start=0, token_count=64)
+    pool.headers.fill(ids, template, [0, 64, 128])
+    assert len(pool.headers) == 3 and ids[1] in pool.headers
+    assert pool.headers[ids[1]] is pool.headers.get(ids[1]) and pool.headers[ids[1]].token_start == 64
+    pool.set_tokens(ids[2], 7)
+    assert pool.headers[ids[2]].token_count == 7 and pool.headers[ids[0]].token_count == 64
+    pool.free(ids[0])
+    assert ids[0] not in pool.headers and sorted(pool.headers) == ids[1:]
+    with pytest.raises(KeyError):
+        pool.headers[ids[0]]
