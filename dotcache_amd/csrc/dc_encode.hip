@@ -17,9 +17,14 @@
 //     from the reciprocal of its group's scale, and from the correctly
 //     rounded division only where that could round differently
 //     (rint_quotients8: the same bits, about 5 instead of 13 instructions
-//     per code).  Taken when the
-//     group size and head_dim are multiples of 8 and the padded head_dim / 8
-//     and group size / 8 are powers of two (every configuration here).
+//     per code).  Taken when head_dim is a multiple of 8, group size / 8 is
+//     a power of two and a padded row fits a wavefront (head_dim 96 or 80
+//     included: 5 rows of 12 lanes, the last 4 lanes idle).  Bound by HBM:
+//     8 x 16384 bf16 tokens of 4 KV heads, float16 keys and 4-bit values,
+//     114 us at head_dim 128 (3.9 TB/s) and 94 us at head_dim 96 (3.6 TB/s),
+//     which took the general kernel 830 us (each thread reads its own
+//     group, 0.4 TB/s); one new token of 64 sequences
+//     14 us against 35.
 //   encode_rows_kernel (the general path): one thread per (row, group),
 //     for any other geometry.
 #include "dc_common.h"
@@ -220,6 +225,18 @@ __device__ __forceinline__ float seg_max(float v, int lanes) {
   return v;
 }
 
+// Maximum over a row's lpr lanes (lane q of the row), in all of them: the
+// butterfly where lpr is a power of two, else every lane visits the row.
+__device__ __forceinline__ float row_max(float v, int lpr, int lane, int q) {
+  if ((lpr & (lpr - 1)) == 0) return seg_max(v, lpr);
+  float m = v;
+  for (int o = 1, p = q; o < lpr; ++o) {
+    p = p + 1 < lpr ? p + 1 : 0;
+    m = fmaxf(m, __shfl(v, lane - q + p, 64));
+  }
+  return m;
+}
+
 // Eight consecutive values of row r from channel c0 (dtype DC_F32 / F16 /
 // BF16); vec: the row start is 16-byte aligned for this dtype.
 template <int32_t dtype, bool vec>
@@ -362,7 +379,7 @@ __device__ __forceinline__ void encode_row(const EncodeJob& J, const float (&x)[
     float am = 0.f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) am = fmaxf(am, fabsf(x[i]));
-    am = seg_max(am, lpr);
+    am = row_max(am, lpr, lane, q);
     const __half s16 = __float2half_rn(fmaxf(am / 127.0f, 1e-8f));
     const float sv = __half2float(s16);
     if (c0 < hd) {
@@ -472,13 +489,15 @@ __global__ void __launch_bounds__(kEncThreads) encode_rows8_kernel(EncodeJob j0,
                                                      rw, c0, g, li, lpr, lpg);
 }
 
-// Whether a pool's geometry fits encode_rows8_kernel: 8-channel lanes that
-// tile its groups and rows within one wavefront, and (2-/3-bit pages) the
-// wavefront's packed words within its LDS share.
+// Whether a pool's geometry fits encode_rows8_kernel: 8-channel lanes, a
+// group's on a power of two of them (its butterfly) and whole rows in one
+// wavefront (rows start at multiples of a group's lanes, so no butterfly
+// crosses a row), and (2-/3-bit pages) the wavefront's packed words within
+// its LDS share.
 static bool fits_rows8(const dc_page_geometry& g) {
   const int32_t G = num_groups(g), Gp = G * g.group_size;
   auto pow2 = [](int32_t v) { return v > 0 && (v & (v - 1)) == 0; };
-  if (g.head_dim % 8 || g.group_size % 8 || !pow2(g.group_size / 8) || !pow2(Gp / 8) || Gp / 8 > 64) return false;
+  if (g.head_dim % 8 || g.group_size % 8 || !pow2(g.group_size / 8) || Gp / 8 > 64) return false;
   // narrow packing: rows per wavefront x words per row <= kPackWords
   const int32_t rpw = 64 / (Gp / 8);
   return int64_t(rpw) * G * words_per_group(g.group_size, 3) <= kPackWords;
@@ -505,7 +524,8 @@ static int encode_launch(const EncodeJob* jobs, int n_jobs, int32_t dtype, int64
     if (!fast[i]) continue;
     const dc_page_geometry& g = jobs[i].pool.geometry;
     const int32_t lpr = num_groups(g) * g.group_size / 8;
-    rows_per_block = rows_per_block < (kEncThreads / lpr) ? rows_per_block : kEncThreads / lpr;
+    const int32_t rows = kEncThreads / 64 * (64 / lpr);  // whole rows per wavefront
+    rows_per_block = rows_per_block < rows ? rows_per_block : rows;
     vec = vec && (reinterpret_cast<uintptr_t>(jobs[i].values) % 16 == 0) && (row_stride * esize) % 16 == 0;
     narrow = narrow || has_narrow(jobs[i].pool);
   }

@@ -139,9 +139,9 @@ def test_encode_rejects_bad_shapes():
 
 # ---- the wavefront encode kernel against the general one and the oracle ----
 
-GEOMS = [  # (head_dim, group_size): the wavefront kernel's shapes and two it leaves to the general kernel
+GEOMS = [  # (head_dim, group_size): the wavefront kernel's shapes and one it leaves to the general kernel
     (128, 32), (64, 32), (256, 32), (128, 64), (48, 32), (32, 16), (128, 128), (64, 8),
-    (96, 32),   # padded head_dim / 8 = 12 lanes: general kernel
+    (96, 32),   # padded head_dim / 8 = 12 lanes, no power of two
     (40, 20),   # group of 20 channels: general kernel
 ]
 FMTS = [("M0", "affine", b) for b in (2, 3, 4, 8)] + [("M0", "symmetric", b) for b in (2, 3, 4, 8)] + [
@@ -334,3 +334,14 @@ def test_encode_rows_kv_equals_two_calls():
                 axis = 1 if name == "payload" else 0
                 np.testing.assert_array_equal(np.take(u, rows, axis=axis).view(np.uint8),
                                               np.take(w, rows, axis=axis).view(np.uint8), err_msg=name)
+
+
+# rows of 12, 10, 20, 5 and 3 lanes (no power of two), with padded channels
+ODD_ROWS = [(96, 32), (80, 16), (160, 32), (40, 8), (24, 8), (72, 32)]
+
+
+@pytest.mark.parametrize("stride_pad", [0, 3])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("hd,gs", ODD_ROWS)
+def test_wavefront_encode_of_rows_off_the_powers_of_two(hd, gs, dtype, stride_pad):
+    test_wavefront_encode_matches_general_kernel_and_oracle(hd, gs, dtype, stride_pad)
