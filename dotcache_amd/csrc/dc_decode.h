@@ -61,8 +61,10 @@ int launch_decode_tiles(const DecodeArgs& a, hipStream_t stream, bool* launched)
 // Launches the MFMA kernel when every format in the pools' masks and the
 // geometry fit it; *launched tells the caller whether to fall back.
 int launch_decode_mfma(const DecodeArgs& a, hipStream_t stream, bool* launched);
-int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_merges, hipStream_t stream,
-                 const dc_window_range* windows = nullptr);
+// n_partials: an upper bound of the partials that the items name in all (picks the
+// launch shape only; a.max_partials bounds what is read).
+int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_merges, int64_t n_partials,
+                 hipStream_t stream, const dc_window_range* windows = nullptr);
 
 // Windows a merge attends (dc_window_merge): at most this many tokens in at
 // most this many pages.

@@ -498,6 +498,106 @@ __global__ void __launch_bounds__(256) merge_kernel(const dc_merge_item* __restr
   }
 }
 
+// One block per (merge item, query head, slice of 4 x kWideCols channels) of
+// kWideRows rows of kWideCols threads: the merge of few streams with many
+// partials each, where merge_kernel's R rows (8 at head_dim 128) walk them
+// one dependent pass after another in a handful of blocks.  The rows'
+// (m_r, l_r, o_r) meet in the wavefront (one maximum, then sums of scaled
+// terms) and the 16 wavefronts' in LDS.  Bound by the latency of its passes
+// (kWideU partials per row each) and of the meeting: one stream's 2048
+// partials of 4 query heads at head_dim 128 (4.2 MB) 52.4 -> 10.0 us, with
+// 8 partials per pass 11.0 (spills at 8 waves per SIMD).
+constexpr int kWideThreads = 1024, kWideCols = 4, kWideRows = kWideThreads / kWideCols, kWideU = 4;
+
+__global__ void __launch_bounds__(kWideThreads, 8) merge_wide_kernel(const dc_merge_item* __restrict__ merges,
+                                                                  const float* part_o, const float* part_ml,
+                                                                  float* out, int32_t n_seqs, int32_t n_kv_heads,
+                                                                  int32_t nq, int32_t hd, int64_t max_partials) {
+  constexpr int kWaves = kWideThreads / 64;
+  __shared__ float4 red[kWaves][kWideCols];
+  __shared__ float2 red_ml[kWaves][kWideCols];
+  const dc_merge_item mi = merges[blockIdx.x];
+  const int j = blockIdx.y, t = threadIdx.x;
+  if (mi.partial_begin < 0 || mi.count <= 0 || int64_t(mi.partial_begin) + mi.count > max_partials) return;
+  if (mi.seq < 0 || mi.seq >= n_seqs || mi.kv_head < 0 || mi.kv_head >= n_kv_heads) return;
+  const int row = t / kWideCols, col = t % kWideCols;
+  const int ch = (int(blockIdx.z) * kWideCols + col) * 4;
+  const bool live = ch < hd;  // (hd is a multiple of 4)
+
+  const float* ml = part_ml + (int64_t(mi.partial_begin) * nq + j) * 2;                    // partial s at ml[2 nq s]
+  const float* po = part_o + (int64_t(mi.partial_begin) * nq + j) * hd + (live ? ch : 0);  // partial s at po[nq hd s]
+  const int64_t mstep = int64_t(nq) * 2, step = int64_t(nq) * hd;
+  float m_r = -INFINITY, l_r = 0.f;
+  float4 acc{0.f, 0.f, 0.f, 0.f};
+  for (int s0 = row; s0 < mi.count; s0 += kWideU * kWideRows) {
+    // a slot past the count loads partial s0 again (always in bounds) and is
+    // masked off, so no load waits on a branch
+    float mv[kWideU], lv[kWideU];
+    float4 xv[kWideU];
+#pragma unroll
+    for (int u = 0; u < kWideU; ++u) {
+      const int s = s0 + u * kWideRows < mi.count ? s0 + u * kWideRows : s0;
+      mv[u] = ml[s * mstep];
+      lv[u] = ml[s * mstep + 1];
+      xv[u] = *reinterpret_cast<const float4*>(po + s * step);
+    }
+    float m_new = m_r;
+#pragma unroll
+    for (int u = 0; u < kWideU; ++u) {
+      if (s0 + u * kWideRows >= mi.count) mv[u] = -INFINITY;
+      m_new = fmaxf(m_new, mv[u]);
+    }
+    if (m_new == -INFINITY) continue;  // every partial so far is empty
+    const float c_old = m_r == -INFINITY ? 0.f : exp2f(m_r - m_new);
+    l_r *= c_old;
+    acc.x *= c_old, acc.y *= c_old, acc.z *= c_old, acc.w *= c_old;
+#pragma unroll
+    for (int u = 0; u < kWideU; ++u) {
+      const float c = mv[u] == -INFINITY ? 0.f : exp2f(mv[u] - m_new);  // an empty partial adds nothing
+      l_r += lv[u] * c;
+      acc.x += xv[u].x * c, acc.y += xv[u].y * c, acc.z += xv[u].z * c, acc.w += xv[u].w * c;
+    }
+    m_r = m_new;
+  }
+
+  // the wavefront's rows: lanes of one column are kWideCols apart
+  float m_w = m_r;
+#pragma unroll
+  for (int o = kWideCols; o < 64; o *= 2) m_w = fmaxf(m_w, __shfl_xor(m_w, o, 64));
+  const float c_r = m_r == -INFINITY ? 0.f : exp2f(m_r - m_w);
+  l_r *= c_r;
+  acc.x *= c_r, acc.y *= c_r, acc.z *= c_r, acc.w *= c_r;
+#pragma unroll
+  for (int o = kWideCols; o < 64; o *= 2) {
+    l_r += __shfl_xor(l_r, o, 64);
+    acc.x += __shfl_xor(acc.x, o, 64);
+    acc.y += __shfl_xor(acc.y, o, 64);
+    acc.z += __shfl_xor(acc.z, o, 64);
+    acc.w += __shfl_xor(acc.w, o, 64);
+  }
+  if ((t & 63) < kWideCols) {
+    red[t >> 6][col] = acc;
+    red_ml[t >> 6][col] = float2{m_w, l_r};
+  }
+  __syncthreads();
+  if (t >= kWideCols || !live) return;
+  float M = -INFINITY, L = 0.f;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) M = fmaxf(M, red_ml[w][col].x);
+  acc = float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    const float2 q = red_ml[w][col];
+    const float c = q.x == -INFINITY ? 0.f : exp2f(q.x - M);
+    const float4 x = red[w][col];
+    L += q.y * c;
+    acc.x += x.x * c, acc.y += x.y * c, acc.z += x.z * c, acc.w += x.w * c;
+  }
+  const float inv = 1.f / fmaxf(L, 1e-30f);
+  float* o = out + ((int64_t(mi.seq) * n_kv_heads + mi.kv_head) * nq + j) * hd + ch;
+  *reinterpret_cast<float4*>(o) = float4{acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+}
+
 int launch_decode_generic(const DecodeArgs& a, hipStream_t stream) {
   bool launched = false;
   if (int rc = launch_decode_tiles(a, stream, &launched); rc || launched) return rc;
@@ -517,15 +617,33 @@ int launch_decode(const DecodeArgs& a, hipStream_t stream) {
   return launched ? DC_OK : launch_decode_generic(a, stream);
 }
 
-int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_merges, hipStream_t stream,
-                 const dc_window_range* windows) {
+int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_merges, int64_t n_partials,
+                 hipStream_t stream, const dc_window_range* windows) {
   if (n_merges <= 0) return DC_OK;
   const int hd = a.kpool.geometry.head_dim;
   // float4 rows when every partial row and output row starts 16-byte aligned
   const bool vec4 = (hd & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.part_o) | reinterpret_cast<uintptr_t>(a.out)) & 15) == 0;
   const int V = vec4 ? 4 : 1;
-  // a whole row per block up to head_dim 128, else slices of 16 x V channels
-  const bool sliced = hd > 128;
+  // Partials per item, and the dependent passes in which a block of whole
+  // rows (up to head_dim 128; 4 partials per row and pass) or of slices (8)
+  // would walk them.
+  const int64_t avg = n_partials / n_merges;
+  const int R = 256 / (hd > 128 ? 16 : hd / V), U = hd > 128 ? 8 : 4;
+  const int64_t passes = (avg + int64_t(R) * U - 1) / (int64_t(R) * U);
+  // The wide blocks where those passes are several and the launch still has
+  // at most one block per CU (at 512 blocks they take turns and lose: 16
+  // query heads of 4 items of 256 partials at head_dim 128, 10.6 -> 9.2 us
+  // wide but 7.5 us sliced).  4 query heads at head_dim 128, 1 / 2 / 4 / 8
+  // items of 2048 partials in all: 52.4 / 27.7 / 15.8 / 9.5 us in whole rows,
+  // 10.0 / 6.5 / 6.3 / 5.6 us wide; 16 items (512 blocks) 6.0 and 6.4; at 2
+  // passes (8 items of 64) 3.5 and 4.0.
+  const dim3 wide_grid(uint32_t(n_merges), uint32_t(a.n_q), uint32_t((hd + 4 * kWideCols - 1) / (4 * kWideCols)));
+  const bool wide = windows == nullptr && vec4 && (passes >= 3 || avg >= 256) &&
+                    int64_t(n_merges) * wide_grid.y * wide_grid.z <= 256;
+  // else a whole row per block up to head_dim 128 and below 256 partials,
+  // and slices of 16 x V channels beyond (16 query heads of 4 items of 512
+  // partials at head_dim 128: 18.9 -> 12.0 us in slices, 16 of 128 11.0 both)
+  const bool sliced = hd > 128 || (windows == nullptr && vec4 && hd >= 64 && avg >= 256);
   const int cols = sliced ? 16 : hd / V;
   const dim3 grid(uint32_t(n_merges), uint32_t(a.n_q), uint32_t((hd / V + cols - 1) / cols));
 #define DC_MERGE(V_, U_, HD_)                                                                                    \
@@ -540,6 +658,9 @@ int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_mer
       DC_MERGE(4, 4, 128);
     else
       DC_MERGE(4, 4, 64);
+  } else if (wide) {
+    hipLaunchKernelGGL(merge_wide_kernel, wide_grid, dim3(kWideThreads), 0, stream, merges, a.part_o, a.part_ml, a.out,
+                       a.n_seqs, a.n_kv_heads, a.n_q, hd, a.max_partials);
   } else if (vec4 && sliced)
     DC_MERGE(4, 8, 0);
   else if (vec4)
@@ -670,7 +791,7 @@ extern "C" int dc_decode_paged_records(dc_pool k_pool, dc_pool v_pool, const int
 
   int rc = dc::launch_decode(a, hipStream_t(stream));
   if (rc) return rc;
-  return dc::launch_merge(a, merges, n_merges, hipStream_t(stream));
+  return dc::launch_merge(a, merges, n_merges, n_partials < n_items ? n_partials : n_items, hipStream_t(stream));
 }
 
 extern "C" int dc_lse_merge(const dc_merge_item* merges, int32_t n_merges, const void* workspace,
@@ -693,7 +814,7 @@ extern "C" int dc_lse_merge(const dc_merge_item* merges, int32_t n_merges, const
   a.part_o = reinterpret_cast<float*>(const_cast<void*>(workspace));
   a.part_ml = a.part_o + n_partials * n_q * head_dim;
   a.max_partials = n_partials;
-  return dc::launch_merge(a, merges, n_merges, hipStream_t(stream));
+  return dc::launch_merge(a, merges, n_merges, n_partials, hipStream_t(stream));
 }
 
 extern "C" int dc_window_merge(dc_pool k_pool, dc_pool v_pool, const int32_t* k_table, const int32_t* v_table,
@@ -737,7 +858,7 @@ extern "C" int dc_window_merge(dc_pool k_pool, dc_pool v_pool, const int32_t* k_
   a.max_partials = n_partials;
   a.recs = records;
   a.rec_stride = records ? dc::kMaxWinPages : 0;
-  return dc::launch_merge(a, merges, n_merges, hipStream_t(stream), windows);
+  return dc::launch_merge(a, merges, n_merges, n_partials, hipStream_t(stream), windows);
 }
 
 extern "C" int32_t dc_decode_waves_per_simd(dc_pool k_pool, dc_pool v_pool, int32_t n_q) {

@@ -342,6 +342,52 @@ def test_lse_merge_matches_float64(hd, layout):
         np.testing.assert_allclose(got[s, h], want, atol=2e-5, rtol=2e-5)
 
 
+# (counts of the 4 items, query heads, head_dim): around the launch rule's
+# lines (128, 256 partials an item; 256 wide blocks) and the wide block's own
+# (256 rows, 1024 partials per pass), odd tails and a partly filled slice
+WIDE_LAYOUTS = [([128, 129, 127, 128], 3, 128), ([256, 255, 257, 256], 1, 64), ([300, 1, 1025, 2050], 2, 96),
+                ([1024, 1, 700, 3], 5, 24), ([256, 260, 250, 258], 16, 128), ([512, 520, 500, 1], 16, 256),
+                ([256, 256, 257, 255], 4, 20)]
+
+
+@pytest.mark.parametrize("counts,nq,hd", WIDE_LAYOUTS)
+def test_lse_merge_of_many_partials_matches_float64(counts, nq, hd):
+    """dc_lse_merge of few streams with many partials each, empty partials at
+    a block's edges and one stream of empty partials only."""
+    import ctypes as C
+
+    import torch
+
+    from dotcache_amd import _lib
+    from dotcache_amd.page_pool import current_stream_ptr
+
+    rng = np.random.default_rng(sum(counts) + hd)
+    n_part = sum(counts)
+    begins = np.cumsum([0] + counts[:-1])
+    part_o = rng.normal(size=(n_part, nq, hd)).astype(np.float32)
+    m = (rng.normal(size=(n_part, nq)) * 8).astype(np.float32)
+    l = rng.uniform(0.5, 40.0, size=(n_part, nq)).astype(np.float32)
+    empty = np.zeros((n_part, nq), bool)
+    empty[:: 7] = True                                             # (every item's first partials among them)
+    empty[begins[3]:begins[3] + counts[3], nq - 1] = True          # one head's item: nothing but empty partials
+    m[empty], l[empty], part_o[empty] = -np.inf, 0.0, 0.0
+    ws = torch.from_numpy(np.concatenate([part_o.ravel(), np.stack([m, l], axis=-1).ravel()])).cuda()
+    items = np.array([[i // 2, i % 2, begins[i], counts[i]] for i in range(4)], np.int32)
+    merges = torch.from_numpy(items.ravel().view(np.uint8).copy()).cuda()
+    out = torch.full((2, 2, nq, hd), 7.0, dtype=torch.float32, device="cuda")
+    _lib.check(_lib.lib().dc_lse_merge(C.c_void_p(merges.data_ptr()), 4, C.c_void_p(ws.data_ptr()), ws.numel() * 4, 2, 2,
+                                       nq, hd, C.c_void_p(out.data_ptr()), C.c_void_p(current_stream_ptr())),
+               "dc_lse_merge")
+    got = out.cpu().numpy()
+    for i, (b, c) in enumerate(zip(begins, counts)):
+        mm = m[b:b + c].astype(np.float64)
+        top = mm.max(axis=0)
+        w = np.where(np.isneginf(mm), 0.0, np.exp2(mm - np.where(np.isneginf(top), 0.0, top)))
+        total = np.sum(w * l[b:b + c], axis=0)
+        want = np.einsum("sq,sqd->qd", w, part_o[b:b + c].astype(np.float64)) / np.maximum(total, 1e-30)[:, None]
+        np.testing.assert_allclose(got[i // 2, i % 2], want, atol=2e-5, rtol=2e-5)
+
+
 @pytest.mark.parametrize("path", ["mfma", "generic"])
 @pytest.mark.parametrize("kfmt,vfmt,vgs", [
     (dict(mode="M3"), dict(bits=4, scheme="symmetric"), 32),   # config 3 formats (keys through LDS)
