@@ -791,6 +791,8 @@ def merge_windows(pool: DevicePagePool, vpool: DevicePagePool, kt: np.ndarray, v
     n = np.asarray(seq_pages, dtype=np.int64)
     page = np.arange(kt.shape[2])
     live = page < n[:, None]
+    # (entries past a sequence's pages may hold anything)
+    kt, vt = np.where(live[:, None, :], kt, 0), np.where(live[:, None, :], vt, 0)
     exact = (pool.formats_of(kt) == f16) & (vpool.formats_of(vt) == f16) & live[:, None, :]
     if not np.all(exact == exact[:, :1]):
         return None

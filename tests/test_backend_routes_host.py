@@ -88,3 +88,11 @@ def test_deferred_headers_are_made_once_and_follow_token_counts():
     assert ids[0] not in pool.headers and sorted(pool.headers) == ids[1:]
     with pytest.raises(KeyError):
         pool.headers[ids[0]]
+
+
+def test_merge_windows_ignore_entries_past_the_pages():
+    k, v = _pool(), _pool()
+    ids = [p.allocate(_lib.FMT_M0_AFFINE, 4, 2, tokens=64) for p in (k, v)]
+    tail = [p.allocate(_lib.FMT_M3_F16, 0, 1, tokens=9) for p in (k, v)]
+    kt, vt = (np.array([[[*i.tolist(), *t.tolist(), 10**6, -7]]]) for i, t in zip(ids, tail))
+    assert merge_windows(k, v, kt, vt, [3]).tolist() == [[2, 3]]
