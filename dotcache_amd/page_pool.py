@@ -23,6 +23,7 @@ from __future__ import annotations
 import ctypes as C
 import functools
 from collections import deque
+from collections.abc import MutableMapping
 from dataclasses import dataclass, replace
 
 import numpy as np
@@ -105,80 +106,54 @@ class PoolGeometry:
         return self._c
 
 
-class _PageHeaders(dict):
+class _PageHeaders(MutableMapping):
     """Page id -> header.  ``fill`` registers the headers of a batch of pages
     that differ in ``token_start`` only; each is made when it is first asked
-    for."""
+    for (by one thread or several: all get the same object)."""
 
     def __init__(self):
-        super().__init__()
+        self._made: dict[int, PageHeader] = {}
         self._deferred: dict[int, tuple[PageHeader, int]] = {}
 
     def discard(self, page_ids: list[int]) -> None:
         """Drop these pages' headers, without making deferred ones."""
-        if self._deferred:
-            for pid in page_ids:
-                self._deferred.pop(pid, None)
-        if dict.__len__(self):
-            for pid in page_ids:
-                dict.pop(self, pid, None)
+        for part in (self._deferred, self._made):
+            if part:
+                for pid in page_ids:
+                    part.pop(pid, None)
 
     def fill(self, page_ids: list[int], template: PageHeader, token_starts: list[int]) -> None:
         self.discard(page_ids)
         self._deferred.update(zip(page_ids, ((template, t) for t in token_starts)))
 
-    def _make(self, pid):
-        template, start = self._deferred.pop(pid)
-        h = replace(template, token_start=start)
-        super().__setitem__(pid, h)
-        return h
-
-    def __setitem__(self, pid, header):
+    def __getitem__(self, pid) -> PageHeader:
+        later = self._deferred.get(pid)
+        if later is None:
+            return self._made[pid]
+        header = self._made.setdefault(pid, replace(later[0], token_start=later[1]))
         self._deferred.pop(pid, None)
-        super().__setitem__(pid, header)
+        return header
 
-    def __missing__(self, pid):
-        if pid in self._deferred:
-            return self._make(pid)
-        raise KeyError(pid)
+    def __setitem__(self, pid, header: PageHeader) -> None:
+        self._made[pid] = header
+        self._deferred.pop(pid, None)
 
-    def get(self, pid, default=None):
-        return self._make(pid) if pid in self._deferred else super().get(pid, default)
+    def __delitem__(self, pid) -> None:
+        if pid not in self:
+            raise KeyError(pid)
+        self.discard([pid])
 
-    def pop(self, pid, *default):
-        if pid in self._deferred:
-            template, start = self._deferred.pop(pid)
-            return replace(template, token_start=start)
-        return super().pop(pid, *default)
-
-    def __contains__(self, pid):
-        return pid in self._deferred or super().__contains__(pid)
-
-    def _all(self):
-        for pid in list(self._deferred):
-            self._make(pid)
+    def __contains__(self, pid) -> bool:
+        return pid in self._deferred or pid in self._made
 
     def __iter__(self):
-        self._all()
-        return super().__iter__()
+        return iter([*self._made, *(pid for pid in self._deferred if pid not in self._made)])
 
-    def keys(self):
-        self._all()
-        return super().keys()
+    def __len__(self) -> int:
+        return len(self._made.keys() | self._deferred.keys())
 
-    def values(self):
-        self._all()
-        return super().values()
-
-    def items(self):
-        self._all()
-        return super().items()
-
-    def __len__(self):
-        return len(self._deferred) + super().__len__()
-
-    def __bool__(self):
-        return len(self) > 0
+    def __bool__(self) -> bool:
+        return bool(self._made) or bool(self._deferred)
 
 
 class DevicePagePool:
@@ -211,7 +186,7 @@ class DevicePagePool:
         # bumped on every descriptor change: page records gathered at one
         # version are stale at any other
         self.desc_version = 0
-        self.headers: dict[int, PageHeader] = _PageHeaders()
+        self.headers: MutableMapping[int, PageHeader] = _PageHeaders()
         self._blob_blocks = np.zeros(self._host_desc.shape[0], dtype=np.int64)  # 256-byte blocks of each live page's blob
         self._live = np.zeros(self._host_desc.shape[0], dtype=bool)
 

@@ -88,6 +88,15 @@ def test_deferred_headers_are_made_once_and_follow_token_counts():
     assert ids[0] not in pool.headers and sorted(pool.headers) == ids[1:]
     with pytest.raises(KeyError):
         pool.headers[ids[0]]
+    # the rest of what a mapping does, on deferred entries too
+    pool.headers.fill(ids[:1], template, [32])
+    assert pool.headers.setdefault(ids[0], None).token_start == 32 and dict(pool.headers) == pool.headers
+    pool.headers.fill(ids[:1], template, [32])
+    del pool.headers[ids[0]]
+    assert ids[0] not in pool.headers and pool.headers.pop(ids[0], None) is None
+    pool.headers.fill(ids[:1], template, [32])
+    pool.headers.clear()
+    assert not pool.headers and list(pool.headers) == []
 
 
 def test_merge_windows_ignore_entries_past_the_pages():
