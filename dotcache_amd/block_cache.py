@@ -101,10 +101,11 @@ class DeviceVllmPagedKVCache:
         self._fill = [np.zeros(n, dtype=np.int32) for _ in range(L)]
         self._final = [np.zeros(n, dtype=bool) for _ in range(L)]
         self._start = [np.full(n, -1, dtype=np.int64) for _ in range(L)]
-        # fp32 rows of the live blocks, [slots, 2, H, P, hd] on the device; live block id -> slot
-        self._row_store = torch.empty((0, 2, H, P, hd), dtype=torch.float32, device=self.device)
+        # fp32 rows of each layer's live blocks, [slots, 2, H, P, hd] on the device; live block id -> slot.
+        # (Per layer: layers may be written on streams of their own.)
+        self._row_store = [torch.empty((0, 2, H, P, hd), dtype=torch.float32, device=self.device) for _ in range(L)]
         self._row_slots = [dict() for _ in range(L)]
-        self._free_slots: list[int] = []
+        self._free_slots: list[list[int]] = [[] for _ in range(L)]
         # the single-sequence view of the reference interface: block ids in token order, cached length
         self._seq_blocks = [[] for _ in range(L)]
         self._seq_len = np.zeros(L, dtype=np.int64)
@@ -158,21 +159,22 @@ class DeviceVllmPagedKVCache:
         self._start[lid][blocks] = -1
         for blk in blocks.tolist():
             if blk in self._row_slots[lid]:
-                self._free_slots.append(self._row_slots[lid].pop(blk))
+                self._free_slots[lid].append(self._row_slots[lid].pop(blk))
 
     def _take_slots(self, lid: int, blocks: list[int]) -> None:
         """An fp32 row slot for every block (the store doubles when none is free)."""
         torch = _torch()
-        short = len(blocks) - len(self._free_slots)
+        store, free = self._row_store[lid], self._free_slots[lid]
+        short = len(blocks) - len(free)
         if short > 0:
-            n = int(self._row_store.shape[0])
+            n = int(store.shape[0])
             m = max(2 * n, n + short)
-            grown = torch.empty((m, *self._row_store.shape[1:]), dtype=torch.float32, device=self.device)
-            grown[:n].copy_(self._row_store)
-            self._row_store = grown
-            self._free_slots.extend(range(m - 1, n - 1, -1))
+            grown = torch.empty((m, *store.shape[1:]), dtype=torch.float32, device=self.device)
+            grown[:n].copy_(store)
+            self._row_store[lid] = grown
+            free.extend(range(m - 1, n - 1, -1))
         for blk in blocks:
-            self._row_slots[lid][blk] = self._free_slots.pop()
+            self._row_slots[lid][blk] = free.pop()
 
     def _allocate_final(self, kind: str, lid: int, n: int) -> np.ndarray:
         """Page ids ``[n, H]`` in the layer's modes."""
@@ -276,7 +278,7 @@ class DeviceVllmPagedKVCache:
         stored = np.asarray([-1 if w else rows[b] for b, w in zip(blk.tolist(), whole.tolist())], dtype=np.int64)[run]
         keep = np.where(stored[:, None] < 0, -1, (stored[:, None] * 2 * H + heads) * P + slot[:, None])
         slots = np.repeat(slot, H)
-        flat = self._row_store.view(-1, hd)
+        flat = self._row_store[lid].view(-1, hd)
         kept = None
         if not whole.all():
             kept = (flat[: flat.shape[0] - H * P], flat[H * P:], keep.ravel())
@@ -293,7 +295,8 @@ class DeviceVllmPagedKVCache:
         P, H, hd = self.block_size, self.num_key_value_heads, self.config.head_dim
         n = len(blocks)
         at = [self._row_slots[lid].pop(b) for b in blocks.tolist()]
-        rows = self._row_store[at[0]][:, None] if n == 1 else self._row_store[torch.as_tensor(at, device=self.device)].transpose(0, 1)
+        store = self._row_store[lid]
+        rows = store[at[0]][:, None] if n == 1 else store[torch.as_tensor(at, device=self.device)].transpose(0, 1)
         new = {}
         for kind in ("K", "V"):
             old = self._map[kind][lid][blocks]
@@ -302,7 +305,7 @@ class DeviceVllmPagedKVCache:
             self._map[kind][lid][blocks] = new[kind]
         tables = torch.from_numpy(np.stack([new["K"], new["V"]]).reshape(2, n * H, 1).astype(np.int32)).to(self.device)
         self.k_pool.encode_streams_with(self.v_pool, rows[0].reshape(n * H, P, hd), rows[1].reshape(n * H, P, hd), tables)
-        self._free_slots.extend(at)
+        self._free_slots[lid].extend(at)
         self._final[lid][blocks] = True
 
     def decode_block_tables(self, layer_id: int, queries, block_tables, context_lens, q_head_to_kv_head=None, *,
