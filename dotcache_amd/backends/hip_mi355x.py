@@ -405,12 +405,15 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
         for i in np.flatnonzero(~score).tolist():
             c = cached[i]
             n = int(offsets[i + 1] - offsets[i])
-            if isinstance(c, torch.Tensor) and c.device.type != "cpu":
+            # (a tensor that requires grad stays one: the logits keep its graph)
+            if isinstance(c, torch.Tensor) and (c.device.type != "cpu" or c.requires_grad):
                 c = c.to(device=dev, dtype=torch.float32)
                 if c.numel() != n:
                     raise ValueError("precomputed page logits must have shape [token_count]")
                 logits[:, offsets[i]: offsets[i + 1]] = c.reshape(1, n)
                 continue
+            if isinstance(c, torch.Tensor):
+                c = c.to(torch.float32).numpy()  # (numpy has no bfloat16)
             c = np.asarray(c, dtype=np.float32).reshape(-1)
             if c.size != n:
                 raise ValueError("precomputed page logits must have shape [token_count]")
@@ -446,7 +449,7 @@ def decode_step_hip(query_slice, key_pages, value_pages, *, precomputed_page_log
     """(logits, weights, output) for one query -- reference ``decode_step_cuda``."""
     q = np.asarray(query_slice, dtype=np.float32) if not hasattr(query_slice, "device") else query_slice
     flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, precomputed_page_logits, trace)
-    logits, weights, out = _split(flat.cpu().numpy(), Q, T, hd)
+    logits, weights, out = _split(flat.detach().cpu().numpy(), Q, T, hd)
     return logits[0].copy(), weights[0].copy(), out[0].copy()
 
 
@@ -455,7 +458,7 @@ def decode_multi_query_step_hip(query_slices, key_pages, value_pages, *, trace: 
     if getattr(q, "ndim", 2) != 2:
         raise ValueError("query_slices must have shape [query_count, head_dim]")
     flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, None, trace)
-    logits, weights, out = _split(flat.cpu().numpy(), Q, T, hd)
+    logits, weights, out = _split(flat.detach().cpu().numpy(), Q, T, hd)
     return logits.copy(), weights.copy(), out.copy()
 
 

@@ -163,3 +163,31 @@ def test_cached_page_logits_are_used_and_their_pages_not_read():
     _, _, out2 = rt.decode_step_with_page_logits(q, kpp, vpp, page_logits=all_cached, backend="hip_mi355x", trace=tr2)
     assert np.max(np.abs(out2 - O.decode_step(q, kp, vp, page_logits=all_cached)[2])) < 1e-3
     assert tr2.payload_bytes_read == sum(p.payload_nbytes for p in vpp)
+
+
+def test_cached_page_logits_of_every_kind_of_tensor():
+    """Cached logits may be lists, arrays or tensors of any float type on
+    either device; one that requires grad stays connected to the logits that
+    the tensor entry point returns."""
+    import torch
+
+    from dotcache_amd import attention_runtime as rt
+    from dotcache_amd.backends.hip_mi355x import decode_multi_query_step_hip_tensor
+
+    rng = np.random.default_rng(1700)
+    hd, n = 64, 64 * 7 + 20
+    kp, vp = ([to_product_page(p) for p in _pages(hard_values(rng, n, hd), 64, hd, kind, bits=4)] for kind in "KV")
+    q = (rng.normal(size=hd) / np.sqrt(hd)).astype(np.float32)
+    # (multiples of 1/8 below 16: the same numbers in every type)
+    want = [(rng.integers(-128, 128, size=p.header.token_count) / 8).astype(np.float32) for p in kp]
+    base = rt.decode_step_with_page_logits(q, kp, vp, page_logits=[*want[:7], None], backend="hip_mi355x")
+    forms = [want[0].tolist(), torch.from_numpy(want[1]).bfloat16(), torch.from_numpy(want[2]).half(),
+             torch.from_numpy(want[3]).double(), torch.from_numpy(want[4]).requires_grad_(),
+             torch.from_numpy(want[5]).bfloat16().cuda(), torch.from_numpy(want[6]).cuda().requires_grad_(), None]
+    got = rt.decode_step_with_page_logits(q, kp, vp, page_logits=forms, backend="hip_mi355x")
+    for a, b in zip(got, base):
+        np.testing.assert_array_equal(a, b)
+    logits, _, out = decode_multi_query_step_hip_tensor(q, kp, vp, precomputed_page_logits=forms)
+    assert torch.equal(out.detach().cpu(), torch.from_numpy(base[2])[None])
+    logits.sum().backward()
+    assert torch.equal(forms[4].grad, torch.ones(64)) and torch.equal(forms[6].grad, torch.ones_like(forms[6]))
