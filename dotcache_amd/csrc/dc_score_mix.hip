@@ -439,42 +439,52 @@ extern "C" int dc_mix_pages_grouped(dc_pool pool, const int32_t* page_ids, const
 namespace dc {
 
 // Softmax of each row (reference attention_reference.py:27-31): exp(x - max)
-// / sum, fp32, one block of 1024 threads per row, from src to dst (which may
-// be the same row).  Up to kSoftmaxRegs columns per thread stay in registers
-// between the passes; longer rows are read again (from dst once the
-// exponentials are there).  Bound by latency at a few thousand columns: one
-// load round, two block reductions (24 rows of 4096: 11.8 -> 4.8 us; 256
-// threads walked the row three times).
+// / sum, fp32, one block of T threads per row, from src to dst (which may be
+// the same row).  Up to kSoftmaxRegs columns per thread stay in registers
+// between the passes (SKIP: columns past the row's end cost no instructions;
+// rows that fill the registers run faster without the branches, 1024 rows of
+// 8192 columns 13.5 us against 14.5); longer rows are read again (from dst
+// once the exponentials are there).  Bound by latency: one load round, two
+// block reductions (24 rows of 4096: 9.9 -> 3.9 us, 8192 rows of 200: 10.2 ->
+// 6.3; 256 threads walked the row three times).
 constexpr int kSoftmaxRegs = 8;
-__global__ void __launch_bounds__(1024) softmax_rows_kernel(const float* src, int64_t src_stride, float* dst,
-                                                            int64_t dst_stride, int32_t n_cols) {
+template <int T, bool SKIP>
+__global__ void __launch_bounds__(T) softmax_rows_kernel(const float* src, int64_t src_stride, float* dst,
+                                                         int64_t dst_stride, int32_t n_cols) {
   const float* x = src + int64_t(blockIdx.x) * src_stride;
   float* y = dst + int64_t(blockIdx.x) * dst_stride;
-  __shared__ float red[2][16];
+  constexpr int kWaves = T / 64;
+  __shared__ float red[2][kWaves];
   const int tid = threadIdx.x;
   float v[kSoftmaxRegs];
+  // (every load of the row in flight: a clamped column, masked)
 #pragma unroll
-  for (int k = 0; k < kSoftmaxRegs; ++k) {  // (every load in flight: a clamped column, masked)
-    const int32_t i = tid + 1024 * k;
+  for (int k = 0; k < kSoftmaxRegs; ++k) {
+    if (SKIP && T * k >= n_cols) break;
+    const int32_t i = tid + T * k;
     v[k] = x[i < n_cols ? i : n_cols - 1];
   }
   float mx = -INFINITY;
 #pragma unroll
-  for (int k = 0; k < kSoftmaxRegs; ++k) mx = tid + 1024 * k < n_cols ? fmaxf(mx, v[k]) : mx;
-  for (int32_t i = tid + 1024 * kSoftmaxRegs; i < n_cols; i += 1024) mx = fmaxf(mx, x[i]);
+  for (int k = 0; k < kSoftmaxRegs; ++k) {
+    if (SKIP && T * k >= n_cols) break;
+    mx = tid + T * k < n_cols ? fmaxf(mx, v[k]) : mx;
+  }
+  for (int32_t i = tid + T * kSoftmaxRegs; i < n_cols; i += T) mx = fmaxf(mx, x[i]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   if (tid % 64 == 0) red[0][tid / 64] = mx;
   __syncthreads();
 #pragma unroll
-  for (int w = 0; w < 16; ++w) mx = fmaxf(mx, red[0][w]);
+  for (int w = 0; w < kWaves; ++w) mx = fmaxf(mx, red[0][w]);
   float sum = 0.f;
 #pragma unroll
   for (int k = 0; k < kSoftmaxRegs; ++k) {
+    if (SKIP && T * k >= n_cols) break;
     v[k] = expf(v[k] - mx);
-    sum += tid + 1024 * k < n_cols ? v[k] : 0.f;
+    sum += tid + T * k < n_cols ? v[k] : 0.f;
   }
-  for (int32_t i = tid + 1024 * kSoftmaxRegs; i < n_cols; i += 1024) {
+  for (int32_t i = tid + T * kSoftmaxRegs; i < n_cols; i += T) {
     const float e = expf(x[i] - mx);
     y[i] = e;
     sum += e;
@@ -485,11 +495,11 @@ __global__ void __launch_bounds__(1024) softmax_rows_kernel(const float* src, in
   __syncthreads();
   sum = 0.f;
 #pragma unroll
-  for (int w = 0; w < 16; ++w) sum += red[1][w];
+  for (int w = 0; w < kWaves; ++w) sum += red[1][w];
 #pragma unroll
   for (int k = 0; k < kSoftmaxRegs; ++k)
-    if (tid + 1024 * k < n_cols) y[tid + 1024 * k] = v[k] / sum;
-  for (int32_t i = tid + 1024 * kSoftmaxRegs; i < n_cols; i += 1024) y[i] = y[i] / sum;
+    if (tid + T * k < n_cols) y[tid + T * k] = v[k] / sum;
+  for (int32_t i = tid + T * kSoftmaxRegs; i < n_cols; i += T) y[i] = y[i] / sum;
 }
 
 }  // namespace dc
@@ -500,8 +510,26 @@ static int softmax_launch(const float* src, int64_t src_stride, float* dst, int6
     return dc::fail(DC_EINVAL, "%s: bad shape", who);
   if (n_rows == 0 || n_cols == 0) return DC_OK;
   if (!src || !dst) return dc::fail(DC_EINVAL, "%s: null pointer", who);
-  hipLaunchKernelGGL(dc::softmax_rows_kernel, dim3(uint32_t(n_rows)), dim3(1024), 0, hipStream_t(stream), src,
-                     src_stride, dst, dst_stride, n_cols);
+#define DC_SOFTMAX(T_, SKIP_)                                                                                        \
+  hipLaunchKernelGGL((dc::softmax_rows_kernel<T_, SKIP_>), dim3(uint32_t(n_rows)), dim3(T_), 0, hipStream_t(stream), \
+                     src, src_stride, dst, dst_stride, n_cols)
+  // The smallest block that loses nothing on few rows: 1024 threads on short
+  // rows leave most of their lanes idle (8192 rows of 200 columns: 34.3 us,
+  // 6.1 in blocks of 64; 4096 of 1000: 21.1, 9.6 in 256; 512 of 2048: 5.2,
+  // 4.3 in 512), and fewer threads wait on more columns each (24 rows of 500:
+  // 3.5 us in 64, 3.0 in 256; of 2048: 3.7 in 256, 3.3 in 512; of 4096: 4.1
+  // in 512, 3.9 in 1024).
+  if (n_cols <= 256)
+    DC_SOFTMAX(64, true);
+  else if (n_cols <= 1024)
+    DC_SOFTMAX(256, true);
+  else if (n_cols <= 2048)
+    DC_SOFTMAX(512, true);
+  else if (n_cols <= 1024 * (dc::kSoftmaxRegs - 1))
+    DC_SOFTMAX(1024, true);
+  else
+    DC_SOFTMAX(1024, false);
+#undef DC_SOFTMAX
   return dc::check_hip(hipGetLastError(), who);
 }
 

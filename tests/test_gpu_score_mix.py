@@ -99,9 +99,10 @@ def test_mix_keeps_infinities_of_valid_rows_only():
     assert np.isposinf(got[5]) and np.isfinite(np.delete(got, 5)).all()
 
 
-@pytest.mark.parametrize("n", [1, 63, 1024, 1025, 8192, 8193, 20000])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 257, 1024, 1025, 2048, 2049, 7168, 7169, 8192, 8193, 20000])
 def test_softmax_rows_in_place_and_out_of_place(n):
-    """Around a row's register columns (8 x 1024) and past them."""
+    """Around the block sizes' lines (256, 1024, 2048 and 7168 columns), a
+    row's register columns (8 x 1024) and past them."""
     import ctypes as C
 
     import torch
@@ -121,3 +122,31 @@ def test_softmax_rows_in_place_and_out_of_place(n):
     assert float(((y - want).abs() / want).max()) < 40 * 2.0 ** -24 + 2e-7 * float((x - x.amax(-1, True)).abs().max())
     assert _lib.lib().dc_softmax_rows(x.data_ptr(), 3, n, n + 5, stream) == 0
     assert torch.equal(x[:, :n], y) and torch.equal(x[:, n:], keep[:, n:])
+
+
+def test_softmax_of_many_short_rows_keeps_its_block_small():
+    """4096 rows of 64 columns take less than three times 64 rows (blocks of
+    1024 threads took seven times as long): both are one round of blocks."""
+    import ctypes as C
+
+    import torch
+
+    from dotcache_amd import _lib
+
+    x = torch.randn((4096, 64), device="cuda")
+    stream = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+    def us(rows):
+        times = []
+        for _ in range(20):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                assert _lib.lib().dc_softmax_rows(x.data_ptr(), rows, 64, 64, stream) == 0
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b) * 50)
+        return sorted(times)[len(times) // 2]
+
+    us(64)
+    assert us(4096) < 3 * us(64)
