@@ -7,7 +7,8 @@
 // The MFMA path for the common formats lives in dc_decode_mfma.hip and is
 // chosen by dc_decode_paged when every page of the call fits it; other pages
 // take dc_decode_tiles.hip, and this kernel only where group_size or head_dim
-// is no multiple of 16.
+// is no multiple of 16 or the tiles do not fit LDS (decode path 1 takes it
+// for every page, to check the other two against).
 //
 // Semantics: reference dotcache/attention_runtime.py:260-315 (concatenate
 // page logits, one softmax over the whole context, mix every value page)
@@ -599,8 +600,6 @@ __global__ void __launch_bounds__(kWideThreads, 8) merge_wide_kernel(const dc_me
 }
 
 int launch_decode_generic(const DecodeArgs& a, hipStream_t stream) {
-  bool launched = false;
-  if (int rc = launch_decode_tiles(a, stream, &launched); rc || launched) return rc;
   hipLaunchKernelGGL(decode_generic_kernel, dim3(uint32_t(a.n_items)), dim3(kThreads), 0, stream, a);
   return check_hip(hipGetLastError(), "decode_generic_kernel launch");
 }
@@ -609,12 +608,12 @@ int launch_decode_generic(const DecodeArgs& a, hipStream_t stream) {
 static int g_decode_path = 0;
 
 int launch_decode(const DecodeArgs& a, hipStream_t stream) {
+  if (g_decode_path == 1) return launch_decode_generic(a, stream);
   bool launched = false;
-  if (g_decode_path != 1)
-    if (int rc = launch_decode_mfma(a, stream, &launched)) return rc;
-  if (!launched && g_decode_path == 2)
-    return fail(DC_EINVAL, "decode path 2: the MFMA kernel does not cover these pools");
-  return launched ? DC_OK : launch_decode_generic(a, stream);
+  if (int rc = launch_decode_mfma(a, stream, &launched); rc || launched) return rc;
+  if (g_decode_path == 2) return fail(DC_EINVAL, "decode path 2: the MFMA kernel does not cover these pools");
+  if (int rc = launch_decode_tiles(a, stream, &launched); rc || launched) return rc;
+  return launch_decode_generic(a, stream);
 }
 
 int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_merges, int64_t n_partials,

@@ -8,8 +8,8 @@
 // partial (m, l, o) for the merge kernel.  Accepted pages: keys M3 fp16 or
 // M0 4- or 8-bit (group 32, affine or symmetric; one width per launch);
 // values M0 4- or 8-bit (group 32 or 64, affine or symmetric) or M3 fp16;
-// up to 16 query heads per KV head.  Other formats take the generic kernel
-// (dc_decode.hip).
+// up to 16 query heads per KV head.  Other formats take the tile kernel
+// (dc_decode_tiles.hip).
 //
 // Prologue: the item, then its pages' table entries, then their
 // descriptors -- or, with page records (dc_gather_page_records), the item

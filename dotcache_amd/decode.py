@@ -673,7 +673,8 @@ _PATHS = {"auto": 0, "generic": 1, "mfma": 2}
 
 
 def set_decode_path(path: str) -> None:
-    """``"auto"`` (MFMA kernel when the pages fit it), ``"generic"``, or
+    """``"auto"`` (the MFMA kernel when the pages fit it, else the tile
+    kernel, else the generic one), ``"generic"`` (that kernel only), or
     ``"mfma"`` (the MFMA kernel only: a decode it does not cover raises
     ValueError)."""
     if path not in _PATHS:

@@ -388,9 +388,9 @@ int dc_gather_page_records(dc_pool k_pool, dc_pool v_pool, const int32_t* k_tabl
 
 /* dc_decode_paged with the page records of its items (from
  * dc_gather_page_records with the same items, tables and descriptors, and
- * the same rec_stride).  The MFMA kernel reads the descriptors of an item
- * of at most rec_stride pages from its records instead of through the
- * tables; other items, and the generic kernel, read the tables.  records
+ * the same rec_stride).  The MFMA and tile kernels read the descriptors of
+ * an item of at most rec_stride pages from its records instead of through
+ * the tables; other items, and the generic kernel, read the tables.  records
  * NULL: exactly dc_decode_paged.  Replaces the same reference functions as
  * dc_decode_paged. */
 int dc_decode_paged_records(dc_pool k_pool, dc_pool v_pool, const int32_t* k_table, const int32_t* v_table,
@@ -460,9 +460,10 @@ int64_t dc_decode_noalloc_scratch_bytes(void);
 /* Process-wide decode kernel choice: 0 (default) runs the MFMA kernel when
  * every page format (M3 fp16 keys and values, M0 4- or 8-bit keys of group
  * 32, M0 4- or 8-bit values of group 32 or 64), head_dim (64/128/256) and
- * n_q <= 16 fit it, and the generic kernel otherwise; 1 always runs the
- * generic kernel (for cross-checking the two); 2 runs only the MFMA kernel
- * and fails with DC_EINVAL where it does not fit (for tests that must know
+ * n_q <= 16 fit it, else the tile kernel when head_dim and both group sizes
+ * are multiples of 16 and a block's tiles fit LDS, and the generic kernel
+ * otherwise; 1 always runs the generic kernel (for cross-checking the other
+ * two); 2 runs only the MFMA kernel and fails with DC_EINVAL where it does not fit (for tests that must know
  * which kernel ran).  Host only; not thread-safe. */
 int dc_set_decode_path(int32_t path);
 

@@ -179,9 +179,9 @@ def test_fused_mixed_key_and_value_formats_every_head_dim(hd, kbits):
             assert err < KERNEL_TOL, f"head block {nqb} pps {pps}: max-abs error {err}"
 
 
-def test_four_and_eight_bit_keys_in_one_pool_take_the_generic_kernel():
+def test_four_and_eight_bit_keys_in_one_pool_leave_the_mfma_kernel():
     """The MFMA kernel takes one key code width per launch: a pool holding
-    both runs on the generic kernel under "auto", and path "mfma" refuses it."""
+    both runs on the tile kernel under "auto", and path "mfma" refuses it."""
     from dotcache_amd.backends import decode_grouped_multiquery_step_prepared_hip_tensor_output_only as fused
     from dotcache_amd.decode import set_decode_path
 

@@ -102,7 +102,7 @@ CASES = [
     (dict(bits=4), dict(bits=8, scheme="symmetric"), 64, 128, 6, 64),
     # head_dim 256, 128-token pages: four chunks per page (config 5 formats)
     (dict(bits=4), dict(bits=4), 32, 256, 4, 128),
-    # 2- and 3-bit codes: the generic kernel only
+    # 2- and 3-bit codes: the tile kernel under "auto"
     (dict(bits=2), dict(bits=3), 32, 64, 3, 96),
 ]
 

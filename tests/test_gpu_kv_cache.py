@@ -95,7 +95,7 @@ def _finalise_contexts(P, T0, steps, T1):
 def test_prefill_append_decode_matches_oracle(page_tokens, case):
     """Prefill of two full pages and a partial tail, then appends one token
     at a time and three at once, across two page finalisations; decode at
-    each stage.  page_tokens 64 runs the MFMA kernel, 16 the generic one."""
+    each stage.  page_tokens 64 runs the MFMA kernel, 16 the tile kernel."""
     import torch
 
     from dotcache_amd.config import DotCacheConfig

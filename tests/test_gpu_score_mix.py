@@ -62,9 +62,12 @@ def test_grouped_logits_weights_and_output(fmt, hd, gs, tpp, Q, lens, layout):
     (160, 32, 32, 64, 1, "token_major"),
 ])
 def test_tile_decode_matches_oracle(kfmt, vfmt, hd, gs, vgs, tpp, Q, layout):
-    """The tile decode over the formats the matrix kernel does not take: token
-    counts of one unit, a partial unit, and several units per wave; one item
-    per group and items of two pages that split a group."""
+    """The tile decode over every pair of formats: token counts of one unit, a
+    partial unit, and several units per wave; one item per group and items of
+    two pages that split a group.  The value pool also holds a 3-bit page that
+    is not read, which keeps the MFMA kernel off the call."""
+    from dotcache_amd import _lib
+    from dotcache_amd.backends import clear_prepared_pools, prepare_pages_hip
     from dotcache_amd.backends import decode_grouped_multiquery_step_prepared_hip_tensor_output_only as fused
     from dotcache_amd.decode import set_decode_path
 
@@ -75,14 +78,72 @@ def test_tile_decode_matches_oracle(kfmt, vfmt, hd, gs, vgs, tpp, Q, layout):
     okp, kp = _groups(rng, hd, gs, kfmt, lens, tpp, "K", layout)
     ovp, vp = _groups(rng, hd, vgs, vfmt, lens, tpp, "V", layout)
     want = O.decode_grouped(q, okp, ovp)
-    set_decode_path("generic")
+    clear_prepared_pools()
+    kp, vp = ([prepare_pages_hip(g) for g in pages] for pages in (kp, vp))
+    for pool in {id(g[0].pool): g[0].pool for g in vp}.values():
+        pool.allocate(_lib.FMT_M0_AFFINE, 3)
+    set_decode_path("mfma")
     try:
-        for pps in (None, 2, 100):
-            got = fused(list(q), kp, vp, pages_per_split=pps).cpu().numpy()
-            # fp32 products and sums on both sides, |out| < 60
-            assert np.max(np.abs(got - want)) < 1e-4, f"pages per split {pps}"
+        with pytest.raises(ValueError, match="MFMA kernel does not cover"):
+            fused(list(q), kp, vp)
+        seen = {}
+        for path in ("auto", "generic"):  # the tile kernel, and the generic kernel on the same pages
+            set_decode_path(path)
+            for pps in (None, 2, 100):
+                seen[path] = got = fused(list(q), kp, vp, pages_per_split=pps).cpu().numpy()
+                # fp32 products and sums on both sides, |out| < 60
+                assert np.max(np.abs(got - want)) < 1e-4, f"{path}, pages per split {pps}"
+        # two kernels: their sums run in different orders and round differently somewhere
+        assert not np.array_equal(seen["auto"], seen["generic"])
     finally:
         set_decode_path("auto")
+        clear_prepared_pools()
+
+
+@pytest.mark.parametrize("kfmt,vfmt", [(FORMATS[i], FORMATS[(3 * i + 1) % len(FORMATS)]) for i in range(len(FORMATS))],
+                         ids=lambda f: "-".join(str(v) for v in f.values()))
+@pytest.mark.parametrize("hd,gs,vgs,tpp,Q,layout", [
+    (48, 24, 24, 64, 4, "group_major"),
+    (40, 20, 40, 32, 3, "token_major"),
+    (30, 32, 32, 64, 1, "group_major"),   # one padded group, rows off 16 bytes
+    (250, 50, 25, 96, 16, "group_major"),
+])
+def test_generic_decode_matches_oracle(kfmt, vfmt, hd, gs, vgs, tpp, Q, layout):
+    """Geometries that 16-channel chunks do not tile have the generic kernel
+    only."""
+    from dotcache_amd.backends import clear_prepared_pools
+    from dotcache_amd.backends import decode_grouped_multiquery_step_prepared_hip_tensor_output_only as fused
+
+    print(f"generic {kfmt} {vfmt} hd {hd} gs {gs}/{vgs} page {tpp} Q {Q} {layout}", flush=True)
+    rng = np.random.default_rng(hd + tpp + Q)
+    lens = [1, 64, tpp + 17, 5 * tpp - 3]
+    q = (rng.normal(size=(len(lens), Q, hd)) / np.sqrt(hd)).astype(np.float32)
+    okp, kp = _groups(rng, hd, gs, kfmt, lens, tpp, "K", layout)
+    ovp, vp = _groups(rng, hd, vgs, vfmt, lens, tpp, "V", layout)
+    want = O.decode_grouped(q, okp, ovp)
+    clear_prepared_pools()
+    for pps in (None, 2):
+        got = fused(list(q), kp, vp, pages_per_split=pps).cpu().numpy()
+        # fp32 products and sums on both sides, |out| < 60
+        assert np.max(np.abs(got - want)) < 1e-4, f"pages per split {pps}"
+
+
+@pytest.mark.parametrize("Q", [8, 9, 16])
+def test_decode_around_the_tiles_lds_limit(Q):
+    """8-bit affine values in 16 groups of 16: 135 KiB of tiles for 8 query
+    heads, 151 KiB for 9 to 16, which the generic kernel takes."""
+    from dotcache_amd.backends import clear_prepared_pools
+    from dotcache_amd.backends import decode_grouped_multiquery_step_prepared_hip_tensor_output_only as fused
+
+    print(f"lds limit Q {Q}", flush=True)
+    rng = np.random.default_rng(Q)
+    lens, hd, tpp = [1, 97, 400], 256, 64
+    q = (rng.normal(size=(len(lens), Q, hd)) / np.sqrt(hd)).astype(np.float32)
+    okp, kp = _groups(rng, hd, 16, dict(bits=4), lens, tpp, "K", "group_major")
+    ovp, vp = _groups(rng, hd, 16, dict(bits=8), lens, tpp, "V", "group_major")
+    clear_prepared_pools()
+    got = fused(list(q), kp, vp).cpu().numpy()
+    assert np.max(np.abs(got - O.decode_grouped(q, okp, ovp))) < 1e-4
 
 
 def test_mix_keeps_infinities_of_valid_rows_only():

@@ -58,7 +58,7 @@ def _noalloc(case, plan, out):
 
 @pytest.mark.parametrize("kfmt,vfmt,hd,Q", [
     (dict(mode="M3"), dict(bits=4, scheme="symmetric"), 128, 7),  # the C3 formats (MFMA kernel)
-    (dict(bits=2), dict(bits=3), 64, 3),                           # generic kernel
+    (dict(bits=2), dict(bits=3), 64, 3),                           # tile kernel
 ])
 def test_noalloc_matches_workspace_decode_twice(kfmt, vfmt, hd, Q):
     import torch
