@@ -62,7 +62,8 @@ int launch_decode_tiles(const DecodeArgs& a, hipStream_t stream, bool* launched)
 // geometry fit it; *launched tells the caller whether to fall back.
 int launch_decode_mfma(const DecodeArgs& a, hipStream_t stream, bool* launched);
 // n_partials: an upper bound of the partials that the items name in all (picks the
-// launch shape only; a.max_partials bounds what is read).
+// launch shape only; a.max_partials bounds what is read).  The entry points take it
+// from workspace_bytes, so hosts pass the plan's bytes and not the buffer's.
 int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_merges, int64_t n_partials,
                  hipStream_t stream, const dc_window_range* windows = nullptr);
 

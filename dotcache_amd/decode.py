@@ -952,6 +952,8 @@ def decode_paged(
     need = workspace_bytes(plan, Q, hd)
     if workspace is None or workspace.numel() < need:
         workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=queries.device)
+    # (the calls below get the plan's bytes, not the buffer's: the merge picks
+    # its launch shape by the partials that the bytes hold)
     if records is not None and not records.fresh_for(plan, k_table, v_table, pool, vpool):
         raise ValueError("page records are stale: gather them again after a change to the plan, the page "
                          "tables or the pools' descriptors")
@@ -972,7 +974,7 @@ def decode_paged(
         m_on = with_merges and merge and plan.merges is not None
         args = (kp, vp, k_table.data_ptr(), v_table.data_ptr(), stride, plan.items.data_ptr() + 32 * first, count,
                 plan.merges.data_ptr() if m_on else None, plan.n_merges if m_on else 0, queries.data_ptr(),
-                dtype_code(queries), float(query_scale), B, H, Q, out.data_ptr(), workspace.data_ptr(), workspace.numel())
+                dtype_code(queries), float(query_scale), B, H, Q, out.data_ptr(), workspace.data_ptr(), need)
         if records is None:
             st = _lib.lib().dc_decode_paged(*args, stream)
         else:
@@ -1009,10 +1011,13 @@ def merge_partials(plan: DecodePlan, out, workspace, *, window=None, records: Pa
     ``window = (pool, v_pool, k_table, v_table, queries, query_scale)`` of
     its decode: the merge attends those pages too (``dc_window_merge``),
     reading their descriptors from ``records`` (``gather_records`` of the
-    plan over those tables) when given."""
+    plan over those tables) when given.  The partials lie where
+    :func:`decode_paged` puts them: in the first ``workspace_bytes(plan,
+    ...)`` bytes, whatever the size of the buffer."""
     if plan.n_merges == 0:
         return
     B, H, Q, hd = (int(x) for x in out.shape)
+    size = min(workspace_bytes(plan, Q, hd), int(workspace.numel()))
     m = np.asarray(plan.host_merges, dtype=np.int64).reshape(-1, 4)
     if np.any((m[:, 0] < 0) | (m[:, 0] >= B)) or np.any((m[:, 1] < 0) | (m[:, 1] >= H)):
         raise ValueError("plan: a merge item names a sequence or KV head outside the output")
@@ -1035,12 +1040,12 @@ def merge_partials(plan: DecodePlan, out, workspace, *, window=None, records: Pa
                                         C.c_void_p(plan.merges.data_ptr()), C.c_void_p(plan.windows.data_ptr()),
                                         plan.n_merges, C.c_void_p(queries.data_ptr()), dtype_code(queries),
                                         float(query_scale), B, H, Q, C.c_void_p(out.data_ptr()),
-                                        C.c_void_p(workspace.data_ptr()), int(workspace.numel()),
+                                        C.c_void_p(workspace.data_ptr()), size,
                                         C.c_void_p(win.data_ptr() if win is not None else 0),
                                         C.c_void_p(current_stream_ptr()))
         _lib.check(st, "dc_window_merge")
         return
     st = _lib.lib().dc_lse_merge(C.c_void_p(plan.merges.data_ptr()), plan.n_merges, C.c_void_p(workspace.data_ptr()),
-                                 int(workspace.numel()), B, H, Q, hd, C.c_void_p(out.data_ptr()),
+                                 size, B, H, Q, hd, C.c_void_p(out.data_ptr()),
                                  C.c_void_p(current_stream_ptr()))
     _lib.check(st, "dc_lse_merge")

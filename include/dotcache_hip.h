@@ -351,7 +351,11 @@ int dc_plan_decode_fill(const int32_t* seq_pages, const int32_t* last_page_token
  *   k_table, v_table : device int32 [n_seqs, n_kv_heads, table_stride] page
  *             ids into k_pool / v_pool
  *   out     : device fp32 [n_seqs, n_kv_heads, n_q, head_dim]
- *   workspace : device, >= dc_decode_workspace_bytes(n_partials, n_q, head_dim)
+ *   workspace : device, workspace_bytes >= dc_decode_workspace_bytes(
+ *             n_partials, n_q, head_dim), and best just that for the
+ *             n_partials of the plan, also where the buffer is larger: the
+ *             bytes say where the partials lie and how many there are at
+ *             most, by which the merge picks its launch shape
  * Replaces reference dotcache/attention_runtime.py:179-315 (decode_step,
  * decode_multi_query_step) and the grouped GPU decode of
  * dotcache/backends/torch_mps.py:4110-4435 behind

@@ -62,6 +62,49 @@ def test_workspace_reused_across_plans():
     _check(wl, 0, [(b, h) for b in range(3) for h in range(H)])
 
 
+@pytest.mark.parametrize("merge", [True, False])
+def test_workspace_size_does_not_change_the_result(merge):
+    """One long stream of 64 partials among 300 whole ones: a kept workspace
+    larger than the plan's partials gives the same bits, with the merge in the
+    decode call or on its own."""
+    import torch
+
+    from dotcache_amd import _lib
+    from dotcache_amd.decode import decode_paged, make_plan, merge_partials, workspace_bytes
+    from dotcache_amd.page_pool import DevicePagePool, PoolGeometry
+
+    hd, P, Q, B, long = 64, 64, 3, 301, 64
+    seq = np.full(B, 1, np.int32)
+    seq[7] = long
+    pools, tables = [], []
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for _ in "KV":
+        pool = DevicePagePool(PoolGeometry(hd, 32, P), reserve_bytes=1 << 22, reserve_pages=512)
+        n = int(seq.sum())
+        ids = pool.allocate(_lib.FMT_M0_AFFINE, 4, n, tokens=P)
+        pool.encode_rows(torch.randn((n * P, hd), generator=gen, device="cuda"), np.repeat(ids, P), np.tile(np.arange(P), n))
+        table = np.zeros((B, 1, long), np.int32)
+        ends = np.cumsum(seq)
+        for b in range(B):
+            table[b, 0, : seq[b]] = ids[ends[b] - seq[b]: ends[b]]
+        pools.append(pool)
+        tables.append(torch.from_numpy(table).cuda())
+    q = torch.randn((B, 1, Q, hd), generator=gen, device="cuda")
+    plan = make_plan(seq, 1, 1, device="cuda")
+    assert plan.n_partials == long and plan.n_merges == 1
+    need = workspace_bytes(plan, Q, hd)
+    outs = []
+    for size in (need, need + 4, 7 * need, 40 * need):
+        ws = torch.zeros(size, dtype=torch.uint8, device="cuda")
+        out = decode_paged(pools[0], *tables, seq, q, plan=plan, workspace=ws, v_pool=pools[1], merge=merge)
+        if not merge:
+            merge_partials(plan, out, ws)
+        outs.append(out)
+    assert torch.isfinite(outs[0]).all()
+    for o in outs[1:]:
+        assert torch.equal(o, outs[0])
+
+
 def test_full_size_c4_sampled_streams():
     """Config 4 at its full shape (64 ragged sequences of 256..32768 tokens,
     per-(layer, KV head) key modes, int8 values, one layer): the longest and
