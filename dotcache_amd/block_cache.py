@@ -102,7 +102,8 @@ class DeviceVllmPagedKVCache:
         self._final = [np.zeros(n, dtype=bool) for _ in range(L)]
         self._start = [np.full(n, -1, dtype=np.int64) for _ in range(L)]
         # fp32 rows of each layer's live blocks, [slots, 2, H, P, hd] on the device; live block id -> slot.
-        # (Per layer: layers may be written on streams of their own.)
+        # (One cache is used from one stream at a time, which a caller that moves to another stream orders:
+        # the layers share the pools' blobs and the workspace.)
         self._row_store = [torch.empty((0, 2, H, P, hd), dtype=torch.float32, device=self.device) for _ in range(L)]
         self._row_slots = [dict() for _ in range(L)]
         self._free_slots: list[list[int]] = [[] for _ in range(L)]
@@ -163,18 +164,39 @@ class DeviceVllmPagedKVCache:
 
     def _take_slots(self, lid: int, blocks: list[int]) -> None:
         """An fp32 row slot for every block (the store doubles when none is free)."""
-        torch = _torch()
-        store, free = self._row_store[lid], self._free_slots[lid]
+        free = self._free_slots[lid]
         short = len(blocks) - len(free)
         if short > 0:
-            n = int(store.shape[0])
+            n = int(self._row_store[lid].shape[0])
             m = max(2 * n, n + short)
-            grown = torch.empty((m, *store.shape[1:]), dtype=torch.float32, device=self.device)
-            grown[:n].copy_(store)
-            self._row_store[lid] = grown
+            self._replace_store(lid, m, n, slice(0, n))
             free.extend(range(m - 1, n - 1, -1))
         for blk in blocks:
             self._row_slots[lid][blk] = free.pop()
+
+    def _replace_store(self, lid: int, slots: int, n: int, rows) -> None:
+        """A row store of ``slots`` slots whose first n hold ``rows`` of the old one."""
+        torch = _torch()
+        store = self._row_store[lid]
+        new = torch.empty((slots, *store.shape[1:]), dtype=torch.float32, device=self.device)
+        if n:
+            new[:n].copy_(store[rows])
+        if store.device.type == "cuda":
+            # (it may have been made on another stream, where its memory could be reused
+            # before this stream has read it)
+            store.record_stream(torch.cuda.current_stream(store.device))
+        self._row_store[lid] = new
+
+    def _shrink_store(self, lid: int) -> None:
+        """Give row slots back: all of them once no block is live, all but twice
+        the live blocks' when fewer than a quarter are in use."""
+        slots = self._row_slots[lid]
+        live = len(slots)
+        if int(self._row_store[lid].shape[0]) <= 4 * live:
+            return
+        self._replace_store(lid, 2 * live, live, list(slots.values()))
+        self._row_slots[lid] = {blk: i for i, blk in enumerate(slots)}
+        self._free_slots[lid] = list(range(2 * live - 1, live - 1, -1))
 
     def _allocate_final(self, kind: str, lid: int, n: int) -> np.ndarray:
         """Page ids ``[n, H]`` in the layer's modes."""
@@ -247,6 +269,7 @@ class DeviceVllmPagedKVCache:
         if restart:
             self._release(lid, restart)
         if not runs:
+            self._shrink_store(lid)
             return
         P, H, hd = self.block_size, self.num_key_value_heads, self.config.head_dim
         blk = np.asarray([r[0] for r in runs], dtype=np.int64)
@@ -287,6 +310,7 @@ class DeviceVllmPagedKVCache:
         done = blk[full & ~whole]
         if done.size:
             self._finalise(lid, done)
+        self._shrink_store(lid)
 
     def _finalise(self, lid: int, blocks: np.ndarray) -> None:
         """Encode full live blocks from their fp32 rows and release their
@@ -512,6 +536,7 @@ class DeviceVllmPagedKVCache:
     def clear_layer(self, layer_id: int) -> None:
         lid = self._check_layer(layer_id)
         self._release(lid, np.flatnonzero((self._map["K"][lid][:, 0] >= 0) | (self._fill[lid] > 0)))
+        self._shrink_store(lid)
         self._seq_blocks[lid] = []
         self._seq_len[lid] = 0
 
