@@ -22,6 +22,7 @@ from __future__ import annotations
 
 import ctypes as C
 import functools
+import threading
 from collections import deque
 from collections.abc import MutableMapping
 from dataclasses import dataclass, replace
@@ -106,54 +107,79 @@ class PoolGeometry:
         return self._c
 
 
+_headers_lock = threading.Lock()
+
+
 class _PageHeaders(MutableMapping):
-    """Page id -> header.  ``fill`` registers the headers of a batch of pages
-    that differ in ``token_start`` only; each is made when it is first asked
-    for (by one thread or several: all get the same object)."""
+    """Page id -> header, with what a dict of them does.  ``fill`` registers
+    the headers of a batch of pages that differ in ``token_start`` only; each
+    is made when it is first asked for (by one thread or several: all get the
+    same object)."""
 
     def __init__(self):
-        self._made: dict[int, PageHeader] = {}
-        self._deferred: dict[int, tuple[PageHeader, int]] = {}
+        self._entries: dict[int, PageHeader | tuple[PageHeader, int]] = {}  # (template, token_start): not made yet
 
     def discard(self, page_ids: list[int]) -> None:
         """Drop these pages' headers, without making deferred ones."""
-        for part in (self._deferred, self._made):
-            if part:
+        with _headers_lock:
+            if self._entries:
                 for pid in page_ids:
-                    part.pop(pid, None)
+                    self._entries.pop(pid, None)
 
     def fill(self, page_ids: list[int], template: PageHeader, token_starts: list[int]) -> None:
         self.discard(page_ids)
-        self._deferred.update(zip(page_ids, ((template, t) for t in token_starts)))
+        with _headers_lock:
+            self._entries.update(zip(page_ids, ((template, t) for t in token_starts)))
 
     def __getitem__(self, pid) -> PageHeader:
-        later = self._deferred.get(pid)
-        if later is None:
-            return self._made[pid]
-        header = self._made.setdefault(pid, replace(later[0], token_start=later[1]))
-        self._deferred.pop(pid, None)
-        return header
+        entry = self._entries[pid]
+        if type(entry) is tuple:
+            with _headers_lock:
+                entry = self._entries[pid]
+                if type(entry) is tuple:
+                    entry = self._entries[pid] = replace(entry[0], token_start=entry[1])
+        return entry
 
     def __setitem__(self, pid, header: PageHeader) -> None:
-        self._made[pid] = header
-        self._deferred.pop(pid, None)
+        with _headers_lock:
+            self._entries[pid] = header
 
     def __delitem__(self, pid) -> None:
-        if pid not in self:
-            raise KeyError(pid)
-        self.discard([pid])
+        with _headers_lock:
+            del self._entries[pid]
 
     def __contains__(self, pid) -> bool:
-        return pid in self._deferred or pid in self._made
+        return pid in self._entries
 
     def __iter__(self):
-        return iter([*self._made, *(pid for pid in self._deferred if pid not in self._made)])
+        return iter(self._entries)
+
+    def __reversed__(self):
+        return reversed(self._entries)
 
     def __len__(self) -> int:
-        return len(self._made.keys() | self._deferred.keys())
+        return len(self._entries)
 
-    def __bool__(self) -> bool:
-        return bool(self._made) or bool(self._deferred)
+    def popitem(self) -> tuple[int, PageHeader]:
+        for pid in reversed(self._entries):
+            return pid, self.pop(pid)
+        raise KeyError("popitem(): no page has a header")
+
+    def copy(self) -> dict[int, PageHeader]:
+        return dict(self)
+
+    def __or__(self, other) -> dict[int, PageHeader]:
+        return self.copy() | other
+
+    def __ror__(self, other) -> dict[int, PageHeader]:
+        return other | self.copy()
+
+    def __ior__(self, other):
+        self.update(other)
+        return self
+
+    def __repr__(self) -> str:
+        return repr(self.copy())
 
 
 class DevicePagePool:

@@ -99,6 +99,35 @@ def test_deferred_headers_are_made_once_and_follow_token_counts():
     assert not pool.headers and list(pool.headers) == []
 
 
+def test_headers_are_a_whole_dict_of_headers():
+    """copy, |, reversed, popitem and the order of a dict, on deferred entries
+    too; reading one moves nothing."""
+    import copy
+    import pickle
+
+    from dotcache_amd.config import DotCacheConfig
+    from dotcache_amd.encode import make_header, resolve_encode_spec
+
+    pool, cfg = _pool(), DotCacheConfig(head_dim=64)
+    template = make_header(cfg, resolve_encode_spec(cfg, kind="K"), kind="K", layer_id=0, kv_head_id=0, token_start=0, token_count=64)
+    ids = pool.allocate(_lib.FMT_M0_AFFINE, 4, 4, tokens=64).tolist()
+    h = pool.headers
+    h.fill(ids[:3], template, [0, 64, 128])
+    h[ids[3]] = template
+    assert h[ids[2]].token_start == 128 and list(h) == ids and list(reversed(h)) == ids[::-1]
+    want = h.copy()
+    assert type(want) is dict and want == h and list(want) == ids and want[ids[1]] is h[ids[1]]
+    assert [p for p in h if h[p].token_start >= 64] == ids[1:3]  # (making entries while iterating)
+    assert h | {99: template} == {**want, 99: template} and {99: template} | h == {99: template, **want}
+    assert repr(h) == repr(want) and copy.deepcopy(h) == want and pickle.loads(pickle.dumps(h)) == want
+    assert h.popitem() == (ids[3], template)
+    h |= {7: template}
+    assert pool.headers is h and h.pop(7) is template and len(h) == 3
+    h.clear()
+    with pytest.raises(KeyError):
+        h.popitem()
+
+
 def test_merge_windows_ignore_entries_past_the_pages():
     k, v = _pool(), _pool()
     ids = [p.allocate(_lib.FMT_M0_AFFINE, 4, 2, tokens=64) for p in (k, v)]
