@@ -279,6 +279,8 @@ class DevicePagePool:
     def allocate(self, fmt: int, bits: int, count: int = 1, *, tokens: int = 0) -> np.ndarray:
         """Allocate ``count`` page blobs of one format; returns int32 page ids.
         Fresh blobs are contiguous, so a batch upload is one copy."""
+        if count < 0:
+            raise ValueError("cannot allocate a negative number of pages")
         nblk = self.blob_bytes(fmt, bits) // 256
         blocks = self._take_blocks(nblk, count)
         ids = self._new_ids(count)

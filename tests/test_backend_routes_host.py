@@ -72,6 +72,15 @@ def test_pool_reuses_blobs_and_ids_in_order():
     assert len(set(many.tolist())) == 40 and (pool.tokens_of(many) == 3).all()
 
 
+def test_a_negative_page_count_is_refused():
+    pool = _pool()
+    a = pool.allocate(_lib.FMT_M0_AFFINE, 4, 2, tokens=64)
+    pool.free(a[:1])
+    with pytest.raises(ValueError):
+        pool.allocate(_lib.FMT_M0_AFFINE, 4, -1)
+    assert pool.n_pages == 2 and pool.allocate(_lib.FMT_M0_AFFINE, 4, 0).size == 0
+
+
 def test_deferred_headers_are_made_once_and_follow_token_counts():
     from dotcache_amd.config import DotCacheConfig
     from dotcache_amd.encode import make_header, resolve_encode_spec
