@@ -451,7 +451,8 @@ class DevicePagePool:
             self._place(new, blocks, [pages[i].header.token_count for i in idx], fmt, bits, nblk)
             ids[idx] = new
             for i, pid in zip(idx, new.tolist()):
-                self.headers[pid] = replace(pages[i].header)
+                h = pages[i].header
+                self.headers[pid] = replace(h) if type(h) is PageHeader else PageHeader.from_dict(h.to_dict())
             if n_old == 0:  # fresh contiguous blocks: one copy
                 self.arena[start * 256: start * 256 + host.size].copy_(src, non_blocking=False)
             else:  # one upload, then a scatter of 256-byte rows into the reused blobs

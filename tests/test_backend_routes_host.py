@@ -137,6 +137,27 @@ def test_headers_are_a_whole_dict_of_headers():
         h.popitem()
 
 
+def test_uploaded_headers_are_page_headers_of_their_own():
+    """Whatever carries the header of an uploaded page, the pool holds a
+    PageHeader with its fields that is not the page's own."""
+    from dataclasses import asdict
+    from types import SimpleNamespace
+
+    from dotcache_amd.config import DotCacheConfig
+    from dotcache_amd.encode import make_header, resolve_encode_spec
+    from dotcache_amd.types import EncodedPage, PageHeader
+
+    cfg = DotCacheConfig(head_dim=64)
+    spec = resolve_encode_spec(cfg, kind="K", mode="M3")
+    plain = make_header(cfg, spec, kind="K", layer_id=3, kv_head_id=1, token_start=64, token_count=2)
+    duck = SimpleNamespace(**asdict(plain))
+    duck.to_dict = lambda: asdict(plain)
+    pool = _pool()
+    for header in (plain, duck):
+        pid = int(pool.upload_pages([EncodedPage(header=header, escape_payload=np.zeros((2, 64), np.float16))])[0])
+        assert type(pool.headers[pid]) is PageHeader and pool.headers[pid] == plain and pool.headers[pid] is not plain
+
+
 def test_merge_windows_ignore_entries_past_the_pages():
     k, v = _pool(), _pool()
     ids = [p.allocate(_lib.FMT_M0_AFFINE, 4, 2, tokens=64) for p in (k, v)]
