@@ -27,6 +27,8 @@
 //     14 us against 35.
 //   encode_rows_kernel (the general path): one thread per (row, group),
 //     for any other geometry.
+#include <stdio.h>
+
 #include "dc_common.h"
 
 namespace dc {
@@ -595,8 +597,11 @@ static int encode_jobs(const dc::EncodeJob* jobs, int n_jobs, int32_t values_dty
   if (values_dtype != DC_F32 && values_dtype != DC_F16 && values_dtype != DC_BF16)
     return dc::fail(DC_EINVAL, "values_dtype must be DC_F32, DC_F16 or DC_BF16");
   if (n_rows == 0) return DC_OK;
-  for (int i = 0; i < n_jobs; ++i)
-    if (int rc = dc::check_encode_args(jobs[i], values_dtype, n_rows, row_stride, who)) return rc;
+  for (int i = 0; i < n_jobs; ++i) {
+    char name[64];
+    snprintf(name, sizeof name, "%s%s", who, n_jobs == 1 ? "" : i == 0 ? " (keys)" : " (values)");
+    if (int rc = dc::check_encode_args(jobs[i], values_dtype, n_rows, row_stride, name)) return rc;
+  }
   return dc::encode_launch(jobs, n_jobs, values_dtype, n_rows, row_stride, hipStream_t(stream));
 }
 
@@ -656,6 +661,7 @@ extern "C" int dc_encode_rows(const void* values, int32_t values_dtype, int64_t 
                               const int32_t* row_page, const int32_t* row_slot, dc_pool pool,
                               dc_stream_t stream) {
   if (int rc = dc::validate_geometry(pool.geometry)) return rc;
+  if (n_rows == 0) return DC_OK;
   const dc::EncodeJob job{values, row_page, row_slot, pool};
   return encode_jobs(&job, 1, values_dtype, n_rows, row_stride, stream, "dc_encode_rows");
 }

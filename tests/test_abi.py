@@ -269,6 +269,22 @@ def test_planner_reports_short_tables():
     assert st == _lib.DC_ESPACE and ni.value == 10 and nm.value == 1
 
 
+def test_encode_argument_checks():
+    """No rows encode nothing, whatever their dtype; an error names the side
+    of a key / value pair that it is about.  (Nothing here reaches a launch.)"""
+    lib = _lib.lib()
+    pool = _lib.Pool(256, 1 << 20, 256, 1, _lib.geometry(64, 32, 16), 0)
+    assert lib.dc_encode_rows(None, 9, 0, 64, None, None, pool, None) == _lib.DC_OK
+    assert lib.dc_encode_rows(256, 9, 1, 64, 256, 256, pool, None) == _lib.DC_EINVAL
+    assert lib.dc_encode_rows(256, 0, -1, 64, 256, 256, pool, None) == _lib.DC_EINVAL
+    assert lib.dc_encode_rows_kv(None, None, 9, 0, 64, None, None, None, None, pool, pool, None) == _lib.DC_EINVAL
+    assert lib.dc_encode_rows_kv(None, None, 0, 0, 64, None, None, None, None, pool, pool, None) == _lib.DC_OK
+    assert lib.dc_encode_rows_kv(256, None, 0, 1, 64, 256, 256, 256, 256, pool, pool, None) == _lib.DC_EINVAL
+    assert b"(values)" in lib.dc_last_error()
+    assert lib.dc_encode_rows_kv(256, 256, 0, 1, 64, 256, None, 256, 256, pool, pool, None) == _lib.DC_EINVAL
+    assert b"(keys)" in lib.dc_last_error()
+
+
 def test_decode_path_switch():
     """Paths 0 (auto), 1 (generic) and 2 (MFMA only) are accepted; anything
     else is DC_EINVAL, and the Python wrapper maps names onto them."""
