@@ -397,8 +397,10 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
     up = _Upload(dev, sid, soff, vid, offsets, *([] if qh is None else [qh]))
     q_ptr = q.data_ptr() if qh is None else up.ptr[4]
     L, stream, base = _lib.lib(), current_stream_ptr(), flat.data_ptr()
+    # (without tokens there are no logits or weights: null, which the library refuses)
+    l_ptr, w_ptr = (base, base + 4 * Q * T) if T else (None, None)
     if sid.size:
-        _lib.check(L.dc_score_pages(kpool.c_pool(), up.ptr[0], up.ptr[1], sid.size, q_ptr, Q, base, T, stream),
+        _lib.check(L.dc_score_pages(kpool.c_pool(), up.ptr[0], up.ptr[1], sid.size, q_ptr, Q, l_ptr, T, stream),
                    "dc_score_pages")
     if not every:
         columns, values = [], []
@@ -422,9 +424,9 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
         if columns:
             logits[:, torch.from_numpy(np.concatenate(columns)).to(dev)] = torch.from_numpy(np.concatenate(values)).to(dev)
     if T:
-        _lib.check(L.dc_softmax_rows_to(base, T, base + 4 * Q * T, T, Q, T, stream), "dc_softmax_rows_to")
-    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, base + 4 * Q * T, Q, T, base + 8 * Q * T, 0,
-                              stream), "dc_mix_pages")
+        _lib.check(L.dc_softmax_rows_to(l_ptr, T, w_ptr, T, Q, T, stream), "dc_softmax_rows_to")
+    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, w_ptr, Q, T, base + 8 * Q * T, 0, stream),
+               "dc_mix_pages")
     return flat, Q, T, int(vpool.geometry.head_dim)
 
 

@@ -191,3 +191,22 @@ def test_cached_page_logits_of_every_kind_of_tensor():
     assert torch.equal(out.detach().cpu(), torch.from_numpy(base[2])[None])
     logits.sum().backward()
     assert torch.equal(forms[4].grad, torch.ones(64)) and torch.equal(forms[6].grad, torch.ones_like(forms[6]))
+
+
+def test_a_step_over_pages_without_tokens_is_refused():
+    """Pages that hold no tokens have no softmax: every step that returns
+    logits refuses them, scored or with (empty) cached logits."""
+    from dotcache_amd import attention_runtime as rt
+    from dotcache_amd.backends.hip_mi355x import decode_multi_query_step_hip_tensor
+
+    rng = np.random.default_rng(1800)
+    kp, vp = (rt.prepare_pages([to_product_page(p) for p in _pages(hard_values(rng, 70, 64), 64, 64, kind, bits=4)])
+              for kind in "KV")
+    for pages in (kp, vp):
+        pages[0].pool.set_tokens([p.page_id for p in pages], 0)
+    q = rng.normal(size=64).astype(np.float32)
+    for step in (lambda: rt.decode_step(q, kp, vp), lambda: rt.decode_multi_query_step(np.stack([q, q]), kp, vp),
+                 lambda: decode_multi_query_step_hip_tensor(q, kp, vp),
+                 lambda: rt.decode_step_with_page_logits(q, kp, vp, page_logits=[[], []])):
+        with pytest.raises(ValueError, match="null pointer"):
+            step()
