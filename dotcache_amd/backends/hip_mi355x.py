@@ -369,10 +369,11 @@ def _pair_pools(key_pages, value_pages, trace):
     return kpool, vpool, kid, vid, kprep + vprep
 
 
-def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits, trace):
-    """(flat, Q, T, head_dim): logits [Q, T], weights [Q, T] and output [Q,
-    head_dim] one after the other in a flat fp32 device tensor (so that one
-    copy takes all three to the host)."""
+def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits, trace, flat: bool = False):
+    """Logits [Q, T], weights [Q, T] and output [Q, head_dim], fp32 on the
+    device: a tensor each (one that is kept does not hold the others), or with
+    ``flat`` one buffer and the shapes ``(buffer, Q, T, head_dim)``, so that
+    one copy takes all three to the host."""
     torch = _torch()
     kpool, vpool, kid, vid, prepared = _pair_pools(key_pages, value_pages, trace)
     kprep, vprep = prepared[:kid.size], prepared[kid.size:]
@@ -391,14 +392,18 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
     qh = _host_queries(query_slices, hd)
     q = _queries_tensor(query_slices, hd, dev) if qh is None else qh
     Q = int(q.shape[0])
-    flat = torch.empty(2 * Q * T + Q * vpool.geometry.head_dim, dtype=torch.float32, device=dev)
-    logits = flat[: Q * T].view(Q, T)
+    vhd = int(vpool.geometry.head_dim)
+    if flat:
+        buffer = torch.empty(2 * Q * T + Q * vhd, dtype=torch.float32, device=dev)
+        logits, weights, out = _split(buffer, Q, T, vhd)
+    else:
+        logits, weights, out = (torch.empty((Q, n), dtype=torch.float32, device=dev) for n in (T, T, vhd))
     sid, soff = (kid, offsets) if every else (kid[score], offsets[:-1][score])
     up = _Upload(dev, sid, soff, vid, offsets, *([] if qh is None else [qh]))
     q_ptr = q.data_ptr() if qh is None else up.ptr[4]
-    L, stream, base = _lib.lib(), current_stream_ptr(), flat.data_ptr()
+    L, stream = _lib.lib(), current_stream_ptr()
     # (without tokens there are no logits or weights: null, which the library refuses)
-    l_ptr, w_ptr = (base, base + 4 * Q * T) if T else (None, None)
+    l_ptr, w_ptr = (logits.data_ptr(), weights.data_ptr()) if T else (None, None)
     if sid.size:
         _lib.check(L.dc_score_pages(kpool.c_pool(), up.ptr[0], up.ptr[1], sid.size, q_ptr, Q, l_ptr, T, stream),
                    "dc_score_pages")
@@ -425,9 +430,9 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
             logits[:, torch.from_numpy(np.concatenate(columns)).to(dev)] = torch.from_numpy(np.concatenate(values)).to(dev)
     if T:
         _lib.check(L.dc_softmax_rows_to(l_ptr, T, w_ptr, T, Q, T, stream), "dc_softmax_rows_to")
-    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, w_ptr, Q, T, base + 8 * Q * T, 0, stream),
+    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, w_ptr, Q, T, out.data_ptr(), 0, stream),
                "dc_mix_pages")
-    return flat, Q, T, int(vpool.geometry.head_dim)
+    return (buffer, Q, T, vhd) if flat else (logits, weights, out)
 
 
 def _split(flat, Q: int, T: int, hd: int):
@@ -443,14 +448,14 @@ def decode_multi_query_step_hip_tensor(query_slices, key_pages, value_pages, *, 
     ``decode_step_with_page_logits``, dotcache/attention_runtime.py:298-303,
     and its device path dotcache/backends/torch_mps.py:2690-2700); the trace
     counts the key pages scored and every value page."""
-    return _split(*_decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits, trace))
+    return _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits, trace)
 
 
 def decode_step_hip(query_slice, key_pages, value_pages, *, precomputed_page_logits=None,
                     trace: ExecutionTrace | None = None) -> tuple[np.ndarray, np.ndarray, np.ndarray]:
     """(logits, weights, output) for one query -- reference ``decode_step_cuda``."""
     q = np.asarray(query_slice, dtype=np.float32) if not hasattr(query_slice, "device") else query_slice
-    flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, precomputed_page_logits, trace)
+    flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, precomputed_page_logits, trace, flat=True)
     logits, weights, out = _split(flat.detach().cpu().numpy(), Q, T, hd)
     return logits[0].copy(), weights[0].copy(), out[0].copy()
 
@@ -459,7 +464,7 @@ def decode_multi_query_step_hip(query_slices, key_pages, value_pages, *, trace: 
     q = np.asarray(query_slices, dtype=np.float32) if not hasattr(query_slices, "device") else query_slices
     if getattr(q, "ndim", 2) != 2:
         raise ValueError("query_slices must have shape [query_count, head_dim]")
-    flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, None, trace)
+    flat, Q, T, hd = _decode_multi(q, key_pages, value_pages, None, trace, flat=True)
     logits, weights, out = _split(flat.detach().cpu().numpy(), Q, T, hd)
     return logits.copy(), weights.copy(), out.copy()
 

@@ -210,3 +210,16 @@ def test_a_step_over_pages_without_tokens_is_refused():
                  lambda: rt.decode_step_with_page_logits(q, kp, vp, page_logits=[[], []])):
         with pytest.raises(ValueError, match="null pointer"):
             step()
+
+
+def test_step_results_hold_their_own_memory():
+    """The logits, weights and output that the tensor entry point returns are
+    three tensors: keeping one does not keep the others."""
+    from dotcache_amd.backends.hip_mi355x import decode_multi_query_step_hip_tensor
+
+    rng = np.random.default_rng(1900)
+    kp, vp = ([to_product_page(p) for p in _pages(hard_values(rng, 200, 64), 64, 64, kind, bits=4)] for kind in "KV")
+    results = decode_multi_query_step_hip_tensor(rng.normal(size=(3, 64)).astype(np.float32), kp, vp)
+    assert [tuple(t.shape) for t in results] == [(3, 200), (3, 200), (3, 64)]
+    for t in results:
+        assert t.storage_offset() == 0 and t.untyped_storage().nbytes() == 4 * t.numel() and t._base is None
