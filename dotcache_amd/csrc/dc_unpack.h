@@ -229,7 +229,6 @@ __device__ __forceinline__ void score_row(const dc_page_desc& d, const dc_page_g
     float q[NB];
     int shift;
   };
-  const float zp = -float((1 << (d.bits - 1)) - 1);
   const bool affine = d.format == DC_FMT_M0_AFFINE;
   Chunk16 ck = chunk16_at(d.format, d.bits, geo, L, 0);
   const uint8_t* row = blob + t * ck.word_step;
@@ -252,6 +251,7 @@ __device__ __forceinline__ void score_row(const dc_page_desc& d, const dc_page_g
     auto dot = [&](const Chunk& x) __attribute__((always_inline)) {
       float v[16], s = 1.f, b = 0.f;
       if constexpr (K != CK_F16 && K != CK_F32) {
+        constexpr float zp = K == CK_B2 ? -1.f : K == CK_B3 ? -3.f : K == CK_B4 ? -7.f : K == CK_B8 ? -127.f : 0.f;
         s = half_bits(x.s, 0);
         b = affine ? half_bits(x.b, 0) : K == CK_I8 ? 0.f : zp * s;
       }
