@@ -164,3 +164,33 @@ def test_merge_windows_ignore_entries_past_the_pages():
     tail = [p.allocate(_lib.FMT_M3_F16, 0, 1, tokens=9) for p in (k, v)]
     kt, vt = (np.array([[[*i.tolist(), *t.tolist(), 10**6, -7]]]) for i, t in zip(ids, tail))
     assert merge_windows(k, v, kt, vt, [3]).tolist() == [[2, 3]]
+
+
+@pytest.mark.parametrize("whole", [0, 8192, 40])
+def test_device_descriptors_follow_the_host_table(whole, monkeypatch):
+    """Both uploads of changed descriptors (by index past ``WHOLE_TABLE_PAGES``
+    pages, the whole table up to it) and the growth of the table."""
+    from dotcache_amd import page_pool
+
+    monkeypatch.setattr(page_pool, "WHOLE_TABLE_PAGES", whole)
+    pool = _pool()
+    rng = np.random.default_rng(whole)
+    live: list[int] = []
+
+    def check():
+        n = pool.n_pages
+        got = pool.device_descs()[:n].numpy().view(page_pool.DESC_DTYPE)
+        np.testing.assert_array_equal(got, pool.descs_of(np.arange(n)))
+        assert got["tokens"][live].min(initial=1) > 0
+
+    for _ in range(30):
+        new = pool.allocate(*((_lib.FMT_M3_F16, 0), (_lib.FMT_M0_AFFINE, 4))[int(rng.integers(2))], int(rng.integers(1, 9)), tokens=5)
+        live += new.tolist()
+        check()
+        pool.set_tokens(rng.choice(live, size=min(3, len(live)), replace=False), int(rng.integers(1, 65)))
+        check()
+        gone = rng.choice(live, size=len(live) // 5, replace=False).tolist()
+        pool.free(gone)
+        live = [p for p in live if p not in gone]
+        check()
+    assert pool.n_pages > 16  # past the table reserved at first
