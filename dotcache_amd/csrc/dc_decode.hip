@@ -506,8 +506,9 @@ __global__ void __launch_bounds__(256) merge_kernel(const dc_merge_item* __restr
 // (m_r, l_r, o_r) meet in the wavefront (one maximum, then sums of scaled
 // terms) and the 16 wavefronts' in LDS.  Bound by the latency of its passes
 // (kWideU partials per row each) and of the meeting: one stream's 2048
-// partials of 4 query heads at head_dim 128 (4.2 MB) 52.4 -> 10.0 us, with
-// 8 partials per pass 11.0 (spills at 8 waves per SIMD).
+// partials of 4 query heads at head_dim 128 (4.2 MB, read from L2) 30.7 -> 5.4
+// us.  Eight partials per pass measured 10 % slower (spills at 8 waves per
+// SIMD).
 constexpr int kWideThreads = 1024, kWideCols = 4, kWideRows = kWideThreads / kWideCols, kWideU = 4;
 
 __global__ void __launch_bounds__(kWideThreads, 8) merge_wide_kernel(const dc_merge_item* __restrict__ merges,
@@ -631,17 +632,21 @@ int launch_merge(const DecodeArgs& a, const dc_merge_item* merges, int32_t n_mer
   const int64_t passes = (avg + int64_t(R) * U - 1) / (int64_t(R) * U);
   // The wide blocks where those passes are several and the launch still has
   // at most one block per CU (at 512 blocks they take turns and lose: 16
-  // query heads of 4 items of 256 partials at head_dim 128, 10.6 -> 9.2 us
-  // wide but 7.5 us sliced).  4 query heads at head_dim 128, 1 / 2 / 4 / 8
-  // items of 2048 partials in all: 52.4 / 27.7 / 15.8 / 9.5 us in whole rows,
-  // 10.0 / 6.5 / 6.3 / 5.6 us wide; 16 items (512 blocks) 6.0 and 6.4; at 2
-  // passes (8 items of 64) 3.5 and 4.0.
+  // query heads of 4 items of 256 partials at head_dim 128, 6.4 us in whole
+  // rows, 7.0 wide and 4.9 sliced).  Kernel times in replayed graphs, 4 query
+  // heads at head_dim 128, 1 / 2 / 4 / 8 items of 2048 partials in all: 30.7 /
+  // 16.9 / 9.8 / 6.2 us in whole rows, 5.4 / 4.7 / 4.8 / 4.9 wide; 16 items
+  // (512 blocks) 4.5 and 5.8.  They begin to win past 96 partials: 8 items of
+  // 64 3.7 us in rows and 4.4 wide, of 96 4.1 and 4.4, of 97 4.6 and 4.5; at
+  // head_dim 64, of 129, 4.6 and 4.4.
   const dim3 wide_grid(uint32_t(n_merges), uint32_t(a.n_q), uint32_t((hd + 4 * kWideCols - 1) / (4 * kWideCols)));
-  const bool wide = windows == nullptr && vec4 && (passes >= 3 || avg >= 256) &&
+  // (Window merges keep merge_kernel, whose blocks hold the window's loads.)
+  const bool wide = windows == nullptr && vec4 && avg > 96 && (passes >= 3 || avg >= 256) &&
                     int64_t(n_merges) * wide_grid.y * wide_grid.z <= 256;
   // else a whole row per block up to head_dim 128 and below 256 partials,
   // and slices of 16 x V channels beyond (16 query heads of 4 items of 512
-  // partials at head_dim 128: 18.9 -> 12.0 us in slices, 16 of 128 11.0 both)
+  // partials at head_dim 128: 9.9 -> 6.4 us in slices; 16 of 128, 4.7 us in
+  // rows and 5.1 in slices)
   const bool sliced = hd > 128 || (windows == nullptr && vec4 && hd >= 64 && avg >= 256);
   const int cols = sliced ? 16 : hd / V;
   const dim3 grid(uint32_t(n_merges), uint32_t(a.n_q), uint32_t((hd / V + cols - 1) / cols));

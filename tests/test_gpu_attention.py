@@ -343,9 +343,9 @@ def test_lse_merge_matches_float64(hd, layout):
 
 
 # (counts of the 4 items, query heads, head_dim): around the launch rule's
-# lines (128, 256 partials an item; 256 wide blocks) and the wide block's own
+# lines (96, 256 partials an item; 256 wide blocks) and the wide block's own
 # (256 rows, 1024 partials per pass), odd tails and a partly filled slice
-WIDE_LAYOUTS = [([128, 129, 127, 128], 3, 128), ([256, 255, 257, 256], 1, 64), ([300, 1, 1025, 2050], 2, 96),
+WIDE_LAYOUTS = [([96, 97, 95, 96], 3, 128), ([97, 98, 96, 97], 3, 128), ([128, 129, 127, 128], 3, 128), ([256, 255, 257, 256], 1, 64), ([300, 1, 1025, 2050], 2, 96),
                 ([1024, 1, 700, 3], 5, 24), ([256, 260, 250, 258], 16, 128), ([512, 520, 500, 1], 16, 256),
                 ([256, 256, 257, 255], 4, 20)]
 
