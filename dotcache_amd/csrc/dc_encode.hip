@@ -20,11 +20,11 @@
 //     per code).  Taken when head_dim is a multiple of 8, group size / 8 is
 //     a power of two and a padded row fits a wavefront (head_dim 96 or 80
 //     included: 5 rows of 12 lanes, the last 4 lanes idle).  Bound by HBM:
-//     8 x 16384 bf16 tokens of 4 KV heads, float16 keys and 4-bit values,
-//     114 us at head_dim 128 (3.9 TB/s) and 94 us at head_dim 96 (3.6 TB/s),
-//     which took the general kernel 830 us (each thread reads its own
-//     group, 0.4 TB/s); one new token of 64 sequences
-//     14 us against 35.
+//     8 x 16384 bf16 tokens of 4 KV heads, float16 keys and affine 4-bit
+//     values, 112.6 us at head_dim 128 (3.9 TB/s) and 87 us at head_dim 96
+//     (3.8 TB/s), which took the general kernel 847 us (each thread reads
+//     its own group, 0.4 TB/s); one new token of 64 sequences 4.4 us against
+//     30.8.
 //   encode_rows_kernel (the general path): one thread per (row, group),
 //     for any other geometry.
 #include <stdio.h>
@@ -431,7 +431,8 @@ __device__ __forceinline__ void encode_row(const EncodeJob& J, const float (&x)[
 // against 170 us for one row block per wavefront in launch order.)
 // EXT: jobs with a table or kept rows; row lists alone take instances without
 // that code (the bulk encode of two lists ran 105.5 us without it and 119.0
-// with it: 8 x 16384 bf16 tokens, 4 KV heads, head_dim 128).
+// with it: 8 x 16384 bf16 tokens, 4 KV heads, head_dim 128, float16 keys and
+// symmetric 4-bit values).
 template <int32_t dtype, bool vec, bool EXT>
 __global__ void __launch_bounds__(kEncThreads) encode_rows8_kernel(EncodeJob j0, EncodeJob j1, int64_t n_rows,
                                                                    int64_t row_stride, int32_t lds_pack) {

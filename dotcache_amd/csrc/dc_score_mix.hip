@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(256) score_pages_kernel(dc_pool pool, const in
 // queries; the next chunks' words fly while one is multiplied.  A launch of a
 // few thousand tokens is bound by its chain of dependent loads (id,
 // descriptor, words).  4096 tokens of 4-bit pages at head_dim 128: one query
-// 37.9 -> 5.6 us, 8 groups of 3 queries 54.8 -> 6.5 us (7.4 and 7.9 with scales
+// 36.6 -> 4.6 us, 8 groups of 3 queries 51.8 -> 5.0 (a third slower with scales
 // converted where they are loaded, which waits for each load).
 template <int NB>
 __global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int32_t* __restrict__ page_ids,
@@ -156,9 +156,9 @@ __global__ void __launch_bounds__(64) score_tiles_kernel(dc_pool pool, const int
 // j's page), and unit j + 1's words are in flight while unit j is summed.
 // One block per slice rather than per query head: a single query's 128
 // channels run on 8 CUs instead of one, 1024 tokens at a time.  4096 tokens of
-// 4-bit pages at head_dim 128: one query 1139 -> 9.4 us, 8 groups of 3
-// queries 1149 -> 10.8 us (8 waves: 14.2 before, and 16.6 us with blocks of 4
-// queries; a third unit in flight does not fit 1024 threads' registers).
+// 4-bit pages at head_dim 128: one query 1135 -> 9.5 us, 8 groups of 3
+// queries 1146 -> 10.8 us (14.2 in 8 waves, 16.6 in blocks of 4 queries; a
+// third unit in flight does not fit 1024 threads' registers).
 template <int QB, int kMixWaves>
 __global__ void __launch_bounds__(64 * kMixWaves) mix_slices_kernel(
     dc_pool pool, const int32_t* __restrict__ page_ids, const int32_t* __restrict__ token_offsets, int32_t n_pages,
@@ -383,7 +383,6 @@ static int mix_launch(const dc_pool& pool, const int32_t* page_ids, const int32_
   if (!weights || !out || (n_pages > 0 && (!page_ids || !token_offsets || !pool.arena || !pool.descs)))
     return dc::fail(DC_EINVAL, "%s: null pointer", who);
   if (dc::chunk16_geometry(pool.geometry) && n_groups <= 65535 && n_queries <= 65535) {
-    // (blocks of as many queries as there are, up to 4: 64 sums per lane)
     // blocks of 2 queries (32 sums per lane) where there are two
     const int qb = n_queries >= 2 ? 2 : 1;
     const dim3 grid(uint32_t(pool.geometry.head_dim / 16), uint32_t((n_queries + qb - 1) / qb), uint32_t(n_groups));
