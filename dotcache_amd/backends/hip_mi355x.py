@@ -395,19 +395,23 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
     vhd = int(vpool.geometry.head_dim)
     if flat:
         buffer = torch.empty(2 * Q * T + Q * vhd, dtype=torch.float32, device=dev)
-        logits, weights, out = _split(buffer, Q, T, vhd)
+        l_ptr = buffer.data_ptr()
+        w_ptr, o_ptr = l_ptr + 4 * Q * T, l_ptr + 8 * Q * T
     else:
         logits, weights, out = (torch.empty((Q, n), dtype=torch.float32, device=dev) for n in (T, T, vhd))
+        l_ptr, w_ptr, o_ptr = logits.data_ptr(), weights.data_ptr(), out.data_ptr()
     sid, soff = (kid, offsets) if every else (kid[score], offsets[:-1][score])
     up = _Upload(dev, sid, soff, vid, offsets, *([] if qh is None else [qh]))
     q_ptr = q.data_ptr() if qh is None else up.ptr[4]
     L, stream = _lib.lib(), current_stream_ptr()
-    # (without tokens there are no logits or weights: null, which the library refuses)
-    l_ptr, w_ptr = (logits.data_ptr(), weights.data_ptr()) if T else (None, None)
+    if T == 0:  # no logits or weights: null, which the library refuses
+        l_ptr = w_ptr = None
     if sid.size:
         _lib.check(L.dc_score_pages(kpool.c_pool(), up.ptr[0], up.ptr[1], sid.size, q_ptr, Q, l_ptr, T, stream),
                    "dc_score_pages")
     if not every:
+        if flat:
+            logits = buffer[: Q * T].view(Q, T)
         columns, values = [], []
         for i in np.flatnonzero(~score).tolist():
             c = cached[i]
@@ -430,7 +434,7 @@ def _decode_multi(query_slices, key_pages, value_pages, precomputed_page_logits,
             logits[:, torch.from_numpy(np.concatenate(columns)).to(dev)] = torch.from_numpy(np.concatenate(values)).to(dev)
     if T:
         _lib.check(L.dc_softmax_rows_to(l_ptr, T, w_ptr, T, Q, T, stream), "dc_softmax_rows_to")
-    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, w_ptr, Q, T, out.data_ptr(), 0, stream),
+    _lib.check(L.dc_mix_pages(vpool.c_pool(), up.ptr[2], up.ptr[3], vid.size, w_ptr, Q, T, o_ptr, 0, stream),
                "dc_mix_pages")
     return (buffer, Q, T, vhd) if flat else (logits, weights, out)
 
